@@ -102,7 +102,9 @@ typedef struct mhcPreExecutor mhcPreExecutor;
  * multiple of 32 from 192 up to 16384, all but small batches) it holds per-team
  * exchange rings only and does not grow with T (7.2 MB at n = 4, D = 7168);
  * the team count is that of the device holding x (of MI355X when the runtime
- * cannot tell).  The two-pass paths hold partial sums that grow with T.
+ * cannot tell).  The two-pass paths hold partial sums that grow with T.  A
+ * shape that runs the slab kernel asks for the larger of its exchange rings
+ * (which do not grow with T) and its path's own layout.
  */
 MHC_API int mhcPreGetWorkspaceSize(const mhcTensor *x, const mhcTensor *phi, const mhcTensor *alpha,
                            const mhcTensor *bias, const mhcTensor *gamma, float normEps,
@@ -144,6 +146,10 @@ MHC_API int mhcPreGetWorkspaceSizeWithHPre(const mhcTensor *x, const mhcTensor *
  * the environment variable MHCPRE_LAUNCH=cooperative at phase 1 the executor
  * uses a cooperative launch, which guarantees co-residency next to concurrent
  * work but dispatches more slowly (about 20 us per launch on MI355X).
+ *
+ * The slab kernel (n = 6) waits between workgroups in the same way, but a
+ * workgroup whose wait expires computes what it waited for itself: such a
+ * launch is slow and its outputs are right, so nothing is reported.
  *
  * A launch may be captured into a HIP graph and replayed: the exchange epoch
  * that tells the current launch's data from stale workspace contents is kept
@@ -256,7 +262,9 @@ MHC_API int mhcPreExecutorSetStatusWord(mhcPreExecutor *executor, uint32_t *devi
 MHC_API const char *mhcPreStatusString(int status);
 
 /* Which kernel path an executor launches (diagnostics and benchmarks):
- * writes a static NUL-terminated name to *name. */
+ * writes a static NUL-terminated name to *name.  The name is that of the
+ * path the shape belongs to: "rows" and "split" shapes with n = 6 run the slab
+ * kernel instead of the path's own kernels where it is faster. */
 MHC_API int mhcPreExecutorPath(const mhcPreExecutor *executor, const char **name);
 
 /*

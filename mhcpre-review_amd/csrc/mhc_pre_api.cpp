@@ -18,6 +18,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstdint>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -90,6 +91,7 @@ struct mhcPreExecutor {
     // device holds x, else at the first launch); -2 until known.
     std::atomic<int> stripCoresident{-2};
     std::atomic<int> fusedCoresident{-2};
+    std::atomic<int> slabCoresident{-2};
     // The caller's sticky device status word (mhcPreExecutorSetStatusWord),
     // or null.
     std::atomic<uint32_t *> statusWord{nullptr};
@@ -222,8 +224,88 @@ StripGeometry strip_geometry(int P, const DeviceShape &s)
     return {1, s.cus, teamsAcross >= 1 ? teamsAcross : mhc::strip_teams_per_xcd(P, s.cus)};
 }
 
+const char *test_env(const char *name);
+
+// How the slab kernel's workgroups (n = 6) divide a device, or P = 0 where no
+// division fits.  A team of P slices needs R reducer workgroups that keep up
+// with it, so the choice is by the time of a team step (one tile), in us, from
+// measurements on MI355X (bf16, gamma, us per launch, groups x teams x R): a
+// slice's own work is 1.45, the reducers' 0.9 + 0.075 P / R, and at least 2
+// with one workgroup.  D = 4096, T = 4096 (32 slices): 1x7x4 71.4, 1x6x4 77.1,
+// 1x6x8 77.6, 1x7x3 77.7, 1x5x8 85.6, 1x7x2 86.7; D = 2048, T = 4096: 1x13x3
+// 43.9, 1x12x4 44.8, 1x14x2 44.9, 1x15x1 55.6, 8x1x4 56.1; D = 1024, T = 8192:
+// 1x25x2 43.8, 8x3x2 43.9, 1x23x3 46.6, 1x28x1 49.8, 8x3x1 52.3, 8x2x4 56.4; D
+// = 512, T = 8192: 1x42x2 30.8, 8x5x2 31.2, 8x4x4 33.8, 8x6x1 34.7.
+mhc::SlabGeometry slab_geometry(int64_t D, int64_t T, const DeviceShape &s)
+{
+    mhc::SlabGeometry best;
+    const int cols = mhc::slab_columns();
+    const int P = static_cast<int>((D + cols - 1) / cols);
+    const int64_t tiles = (T + 15) / 16;
+    double bestTime = 0.0;
+    const auto consider = [&](int groups, int teams, int R) {
+        const int perGroup = s.cus / groups;
+        if (teams < 1 || R < 1 || (P + R) * teams > perGroup) {
+            return;
+        }
+        // Waves: CC for the hPre columns and 3 CR for the others.
+        const int CC = R >= 4 ? 8 : R >= 2 ? 4 : 2;
+        const int CR = std::min(8, (8 * R - CC) / 3);
+        const double load = static_cast<double>(P) / R;
+        const double step = std::max(R == 1 ? 2.0 : 1.45, 0.9 + 0.075 * load);
+        const int64_t all = static_cast<int64_t>(groups) * teams;
+        const double time = static_cast<double>((tiles + all - 1) / all) * step;
+        if (best.P == 0 || time < bestTime * 0.999) {
+            bestTime = time;
+            best = {P, groups, teams, R, CC, CR, s.cus, s.xcds};
+        }
+    };
+    const char *force = test_env("MHCPRE_SLAB");
+    int f[3];
+    if (force != nullptr && std::sscanf(force, "%d,%d,%d", &f[0], &f[1], &f[2]) == 3 &&
+        (f[0] == 1 || f[0] == s.xcds)) {
+        consider(f[0], f[1], f[2]);
+        return best;
+    }
+    for (const int groups : {s.xcds, 1}) {
+        const int perGroup = s.cus / groups;
+        for (int teams = perGroup / (P + 1); teams >= 1; --teams) {
+            consider(groups, teams, std::min(8, perGroup / teams - P));
+        }
+        if (s.xcds == 1) {
+            break;
+        }
+    }
+    return best;
+}
+
+// Where the slab kernel is faster than the kernels of its shape's path (n = 6).
+// Measured on MI355X (bf16, gamma, back to back, us, slab / the rows or split
+// path): K % 128 == 0: D = 256, T = 2048 15.6 / 15.0, 4096 17.1 / 18.6; D =
+// 768, T = 256 14.6 / 12.8, 512 15.0 / 16.8; D = 1024, T = 512 15.1 / 15.5,
+// 2048 22.0 / 25.8, 8192 43.8 / 62.6; D = 2048, T = 512 19.0 / 18.9, 768 19.6
+// / 21.3, 4096 44.7 / 60.0; D = 4096, T = 512 23.8 / 23.4, 768 25.8 / 28.4,
+// 4096 73.9 / 96.7; D = 5120, T = 1024 41.2 / 37.2, 2048 59.8 / 63.5; D =
+// 6144, T = 2048 69.1 / 70.3, 4096 119.6 / 125.7; D = 8192, T = 2048 90.6 /
+// 85.2; fp16 D = 1024, T = 512 16.5 / 16.5, D = 4096, T = 4096 82.0 / 100.3;
+// prepared weights gain 3 us more.  Other widths (the split path, three
+// launches): D = 272, T = 8192 29.1 / 28.2; D = 400 32.7 / 34.6; D = 1040, T =
+// 64 15.1 / 14.5, 1500 24.3 / 23.1, 4096 36.7 / 40.0; D = 1200, T = 777 19.1 /
+// 19.3; D = 2000, T = 1 15.4 / 16.2, 2048 33.3 / 39.4, 8192 88.1 / 139.1; D =
+// 4880, T = 8 19.6 / 27.5, 4096 114.7 / 170.6; D = 8176, T = 4096 182 / 285.
+bool slab_faster(int64_t D, int64_t T)
+{
+    if ((6 * D) % 128 != 0) {
+        return D >= 1600 || (D >= 960 && T >= 4096) || (D >= 400 && T >= 8192);
+    }
+    if (D < 256) {
+        return false;
+    }
+    return T >= (D <= 640 ? 4096 : D <= 1536 ? 512 : D <= 4096 ? 768 : D <= 6144 ? 2048 : kMaxRows);
+}
+
 // Phase-1 knobs for tests and measurement sweeps (MHCPRE_FORCE_PATH,
-// MHCPRE_SPIN_LIMIT, MHCPRE_ROWS_B, MHCPRE_ROWS_PARTIALS) are read only when
+// MHCPRE_SPIN_LIMIT, MHCPRE_ROWS_B, MHCPRE_ROWS_PARTIALS, MHCPRE_SLAB) are read only when
 // MHCPRE_TESTING=1: a stray one in a production environment changes nothing.
 const char *test_env(const char *name)
 {
@@ -677,6 +759,19 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
         }
     }
     const char *force = test_env("MHCPRE_FORCE_PATH");
+    // Slab kernel (n = 6), in place of the rows or split path's kernels.
+    const bool slabForced = force != nullptr && std::strcmp(force, "slab") == 0;
+    if (n == 6 && (slabForced || (force == nullptr && slab_faster(D, T))) &&
+        D <= mhc::slab_max_slices() * mhc::slab_columns() && T < (int64_t{1} << 24)) {
+        DeviceShape shape = kPlanShapeDefault;
+        if (planDevice < 0 || !device_shape_of(planDevice, shape)) {
+            (void)hipGetLastError();
+            shape = kPlanShapeDefault;
+        }
+        if (shape.cus <= mhc::kMaxEpochGrid) {
+            p.slab = slab_geometry(D, T, shape);
+        }
+    }
     if (force != nullptr) {
         if (std::strcmp(force, "split") == 0) {
             p.path = mhc::Path::kSplit;
@@ -774,6 +869,24 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
     default:
         p.wsTotal = splitEnd;
         break;
+    }
+    if (p.slab.P > 0) {
+        const size_t slots = static_cast<size_t>(p.slab.groups) * p.slab.teams * mhc::slab_ring_slots();
+        p.wsSlabBcast = mhc::kWsHeaderBytes;
+        p.wsSlabFlags = align_up(p.wsSlabBcast + slots * mhc::slab_bcast_words() * 8, 256);
+        p.wsSlabDone = align_up(p.wsSlabFlags + slots * p.slab.P * 2 * 8, 256);
+        p.wsSlabRecs = align_up(p.wsSlabDone + static_cast<size_t>(p.slab.groups) * p.slab.teams *
+                                                   mhc::slab_done_words() * 8,
+                                256);
+        const size_t slabEnd =
+            align_up(p.wsSlabRecs + slots * p.slab.P * mhc::slab_record_words() * 8, 256);
+        // Not where it would take a call past the built-in scratch that the
+        // other kernels' layout fits.
+        if (slabEnd > mhc::kScratchBytes && p.wsTotal <= mhc::kScratchBytes) {
+            p.slab = mhc::SlabGeometry{};
+        } else {
+            p.wsTotal = std::max(p.wsTotal, slabEnd);
+        }
     }
     if (useCache) {
         std::lock_guard<std::mutex> lock(plan_cache_mutex());
@@ -909,7 +1022,7 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     // error an earlier call of the process may have left there (the split
     // path makes no other HIP call before its first launch).
     (void)hipGetLastError();
-    if (p.path != mhc::Path::kSplit && !device_shape(device, shape)) {
+    if ((p.path != mhc::Path::kSplit || p.slab.P > 0) && !device_shape(device, shape)) {
         return MHC_STATUS_HIP_ERROR;
     }
     const uint32_t launchId = next_launch_id();
@@ -965,6 +1078,11 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
             done = true;
         }
     }
+    if (!done && p.slab.P > 0 && p.slab.grid == shape.cus && p.slab.xcds == shape.xcds &&
+        cached_coresident(executor->slabCoresident, mhc::slab_max_coresident, p, shape.cus) >= shape.cus) {
+        err = mhc::launch_slab(p, workspace, stream);
+        done = true;
+    }
     if (!done && p.path == mhc::Path::kRows) {
         err = mhc::launch_rows(p, workspace, shape.xcds, stream);
         done = true;
@@ -997,6 +1115,9 @@ void prime_coresident(mhcPreExecutor *ex)
     void *scratch = nullptr;
     if (mhc::scratch_address(device, &scratch) != hipSuccess) {
         (void)hipGetLastError();
+    }
+    if (p.slab.P > 0) {
+        (void)cached_coresident(ex->slabCoresident, mhc::slab_max_coresident, p, shape.cus);
     }
     if (p.path != mhc::Path::kStrip && p.path != mhc::Path::kFused) {
         return;

@@ -4,6 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "mhc_pre.h"
 
 namespace mhc {
@@ -162,6 +165,96 @@ __device__ __forceinline__ bf16x8_t as_bf16x8(const u32x4_t &v) { return __built
 __device__ __forceinline__ f32x4_t mfma16(const u32x4_t &a, const u32x4_t &b, const f32x4_t &c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
+}
+
+// Cache policies of the buffer instructions below.
+constexpr int kCpolNt = 2;    // nontemporal: streamed once
+constexpr int kCpolDev = 16;  // sc1: device scope, written through, read past the L1 and L2 of another XCD
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, int bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, bytes, 0x00020000);
+}
+
+template <int kCpol>
+__device__ __forceinline__ u32x4_t load16(__amdgpu_buffer_rsrc_t r, int off)
+{
+    return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kCpol));
+}
+
+template <int kCpol>
+__device__ __forceinline__ void store16(const u32x4_t &v, __amdgpu_buffer_rsrc_t r, int off)
+{
+    __builtin_amdgcn_raw_buffer_store_b128(
+        __builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned int, v), r, off, 0, kCpol);
+}
+
+// Waits until at most `kOut` of this wave's vector-memory loads are still in
+// flight (they complete in issue order), without waiting on LDS or exports.
+template <int kOut>
+__device__ __forceinline__ void wait_vm()
+{
+    static_assert(kOut >= 0 && kOut < 64, "vmcnt range");
+    // s_waitcnt fields: vmcnt [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8].
+    constexpr int imm = (kOut & 15) | ((kOut >> 4) << 14) | (7 << 4) | (15 << 8);
+    __builtin_amdgcn_s_waitcnt(imm);
+}
+
+// Workgroup barrier that orders LDS only (no wait for outstanding global
+// accesses, which __syncthreads() would add).
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Calls f(std::integral_constant<int, i>{}) for i = 0 .. kCount-1.
+template <typename F, int... kIs>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, kIs...>)
+{
+    (f(std::integral_constant<int, kIs>{}), ...);
+}
+template <int kCount, typename F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    static_for_seq(f, std::make_integer_sequence<int, kCount>{});
+}
+
+// A fragments of k-steps 2q and 2q + 1 from line-layout registers r0 (rows
+// 0-7) and r1 (rows 8-15).  In a line register lane l holds row l & 7 and the
+// 8 columns at 8(l >> 4) + 32((l >> 3) & 1) of a 64-column line; the A
+// fragment wants row l & 15 and columns 8(l >> 4) of its k-step, so lanes
+// with bit 3 set take the other register's lane l ^ 8 (DPP row_ror:8 with
+// banks 2-3 or 0-1 enabled).
+__device__ __forceinline__ void lines_to_frags(const u32x4_t &r0, const u32x4_t &r1, u32x4_t &k0,
+                                               u32x4_t &k1)
+{
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        k0[w] = (uint32_t)__builtin_amdgcn_update_dpp((int)r0[w], (int)r1[w], 0x128, 0xF, 0xC, false);
+        k1[w] = (uint32_t)__builtin_amdgcn_update_dpp((int)r1[w], (int)r0[w], 0x128, 0xF, 0x3, false);
+    }
+}
+
+// One of the two.
+template <int kStep>
+__device__ __forceinline__ u32x4_t line_frag(const u32x4_t &r0, const u32x4_t &r1)
+{
+    u32x4_t k;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        k[w] = kStep == 0 ? (uint32_t)__builtin_amdgcn_update_dpp((int)r0[w], (int)r1[w], 0x128, 0xF, 0xC, false)
+                          : (uint32_t)__builtin_amdgcn_update_dpp((int)r1[w], (int)r0[w], 0x128, 0xF, 0x3, false);
+    }
+    return k;
+}
+
+__device__ __forceinline__ f32x4_t mfma16_f16(const u32x4_t &a, const u32x4_t &b, const f32x4_t &c)
+{
+    typedef _Float16 f16x8_t __attribute__((__vector_size__(8 * sizeof(_Float16))));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
 
 // fp16 x -> exact bf16 pair: x = hi + lo (an fp16 significand has 11 bits).

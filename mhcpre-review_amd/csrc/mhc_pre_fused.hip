@@ -150,15 +150,6 @@ __device__ __forceinline__ uint64_t ld_word(const uint64_t *p)
     return __hip_atomic_load(const_cast<uint64_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Cache-policy operands of the buffer builtins.
-constexpr int kCpolNt = 2;    // nontemporal: x and hIn are streamed once
-constexpr int kCpolDev = 16;  // sc1: device-scope coherent
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, int bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, bytes, 0x00020000);
-}
-
 // Sums over the P slice records of a tile, for record columns c0 .. c0+NC-1
 // and all 16 rows, checking every word's tag.  Lane l takes item
 // it = l % (8 NC) (column c0 + it/8, rows 2(it%8) and 2(it%8) + 1, one 16-byte
@@ -211,26 +202,6 @@ __device__ __forceinline__ float2 sum_records(__amdgpu_buffer_rsrc_t r, int c0, 
     }
     valid = __all(ok);
     return tot;
-}
-
-// A fragments of k-steps 2kp and 2kp + 1 from the line-layout registers r0
-// (rows 0-7) and r1 (rows 8-15): lanes with bit 3 set take the other
-// register's lane l ^ 8 (DPP row_ror:8 with banks 2-3 or 0-1 enabled).
-__device__ __forceinline__ void lines_to_frags(const u32x4_t &r0, const u32x4_t &r1, u32x4_t &k0,
-                                               u32x4_t &k1)
-{
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        k0[w] = (uint32_t)__builtin_amdgcn_update_dpp((int)r0[w], (int)r1[w], 0x128, 0xF, 0xC, false);
-        k1[w] = (uint32_t)__builtin_amdgcn_update_dpp((int)r1[w], (int)r0[w], 0x128, 0xF, 0x3, false);
-    }
-}
-
-__device__ __forceinline__ f32x4_t mfma16_f16(const u32x4_t &a, const u32x4_t &b, const f32x4_t &c)
-{
-    typedef _Float16 f16x8_t __attribute__((__vector_size__(8 * sizeof(_Float16))));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
 
 __device__ __forceinline__ void record_timeout(const FusedArgs &a, int lane)

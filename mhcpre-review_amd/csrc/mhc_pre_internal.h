@@ -35,6 +35,18 @@ constexpr size_t kWsSeenOff = 256;            // uint32 [kMaxEpochGrid]: epoch e
 constexpr int kMaxEpochGrid = 2048;           // largest strip / fused grid
 constexpr size_t kWsHeaderBytes = kWsSeenOff + 4 * kMaxEpochGrid;
 
+// Work distribution of the slab kernel (mhc_pre_slab.hip).
+struct SlabGeometry {
+    int P = 0;       // slice workgroups per team
+    int groups = 0;  // XCDs (teams inside an XCD), or 1 (teams across the device)
+    int teams = 0;   // teams per group
+    int R = 0;       // reducer workgroups per team
+    int CC = 0;      // reducer waves of the hPre columns (1, 2, 4 or 8)
+    int CR = 0;      // reducer waves of each block of the other columns (up to 8)
+    int grid = 0;    // workgroups: one per CU
+    int xcds = 0;    // XCDs of the device it was planned for
+};
+
 struct Plan {
     Path path = Path::kSplit;
 
@@ -88,6 +100,11 @@ struct Plan {
     int stripTeamsPerXcd = 0;
     int stripGrid = 0;
 
+    // Slab kernel (n = 6; slab.P == 0: not taken): one launch that runs in place of
+    // the rows or split path's kernels, whose layout the workspace also holds
+    // (the fallback on a device that cannot co-schedule its grid).
+    SlabGeometry slab;
+
     // Rows path (K % 128 == 0): rowsS K-ranges (contiguous runs of
     // rows_stage_ksteps()-k-step stages) over rowsBlocks blocks of
     // rows_block_rows() rows.
@@ -116,6 +133,10 @@ struct Plan {
     size_t wsStripRecs = 0;   // strip: per-team rings of P exchange records (tagged words)
     size_t wsRowsB = 0;       // rows (prep launch): B fragments [K/32][NT][64 lanes] x 16 bytes
     size_t wsRowsPartial = 0; // rows: partials, [rowsS][T][M+1] or [T][rowsS][M+1]
+    size_t wsSlabBcast = 0;   // slab: per-team rings of broadcast blocks
+    size_t wsSlabFlags = 0;   // slab: per-team rings of the slices' flags
+    size_t wsSlabDone = 0;    // slab: the reducer waves' done words
+    size_t wsSlabRecs = 0;    // slab: per-team rings of P exchange records
     size_t wsTotal = 0;
 
     // Bound device pointers (caller memory).
@@ -148,6 +169,16 @@ hipError_t launch_split(const Plan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_fused(const Plan &plan, void *workspace, uint32_t launchId, hipStream_t stream);
 
 hipError_t launch_strip(const Plan &plan, void *workspace, uint32_t launchId, hipStream_t stream);
+
+// Slab kernel (mhc_pre_slab.hip): one launch, x read once.
+hipError_t launch_slab(const Plan &plan, void *workspace, hipStream_t stream);
+int slab_max_coresident(const Plan &plan, int numCUs);
+int slab_columns();                          // x columns per slice
+int slab_max_slices();                       // largest P
+int slab_done_words();                       // words of a team's done array
+int slab_ring_slots();                       // exchange ring slots per team
+int slab_record_words();                     // tagged 8-byte words of a record
+int slab_bcast_words();                      // ... and of a broadcast block
 
 // Prepared B operand (mhc_pre_rows.hip): B = gamma (.) phi (gamma may be
 // null) split into bf16 hi + lo MFMA fragments, [K/32 k-steps][2M/16 column

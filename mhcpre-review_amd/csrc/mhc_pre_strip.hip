@@ -61,9 +61,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <mutex>
 #include <type_traits>
-#include <utility>
 
 namespace mhc {
 namespace {
@@ -182,14 +180,6 @@ __device__ __forceinline__ uint32_t bcast_tag(uint32_t pos, uint32_t epoch)
     return (pos * 0x85EBCA77u) ^ epoch ^ 0xC2B2AE3Du;
 }
 
-constexpr int kCpolNt = 2;    // nontemporal: x and hIn are streamed once
-constexpr int kCpolDev = 16;  // sc1: device-scope coherent
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, int bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, bytes, 0x00020000);
-}
-
 // Every global access of the kernel is a buffer instruction, the exchange
 // words and the status word included (aligned 8-byte accesses, performed as
 // one access, sc1).  Atomics through generic pointers would compile to FLAT
@@ -207,40 +197,12 @@ __device__ __forceinline__ void st_status(uint64_t *status, uint32_t launchId)
                                           make_rsrc(status, 8), 0, 0, kCpolDev);
 }
 
-template <int kCpol>
-__device__ __forceinline__ void store16(const u32x4_t &v, __amdgpu_buffer_rsrc_t r, int off)
-{
-    __builtin_amdgcn_raw_buffer_store_b128(
-        __builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned int, v), r, off, 0, kCpol);
-}
-
 __device__ __forceinline__ void record_timeout(const StripArgs &a, int lane)
 {
     if (lane == 0) {
         st_status(reinterpret_cast<uint64_t *>(a.hdr), a.launchId);
         st_status_word(a.statusWord);
     }
-}
-
-// Calls f(std::integral_constant<int, i>{}) for i = 0 .. kCount-1.
-template <typename F, int... kIs>
-__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, kIs...>)
-{
-    (f(std::integral_constant<int, kIs>{}), ...);
-}
-template <int kCount, typename F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    static_for_seq(f, std::make_integer_sequence<int, kCount>{});
-}
-
-// Workgroup barrier that orders LDS only.  __syncthreads() also makes every
-// outstanding global load and store of the wave complete first.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Workgroup-wide AND of ok through LDS, with a barrier that orders LDS only
@@ -262,26 +224,6 @@ __device__ __forceinline__ bool wg_all(bool ok, uint32_t *votes, uint32_t &parit
     const u32x4_t v0 = v[0];
     const u32x4_t v1 = v[1];
     return (v0[0] & v0[1] & v0[2] & v0[3] & v1[0] & v1[1] & v1[2] & v1[3]) != 0u;
-}
-
-// A fragments of k-steps 2q and 2q + 1 from the line-layout registers r0
-// (rows 0-7) and r1 (rows 8-15): lanes with bit 3 set take the other
-// register's lane l ^ 8 (DPP row_ror:8 with banks 2-3 or 0-1 enabled).
-__device__ __forceinline__ void lines_to_frags(const u32x4_t &r0, const u32x4_t &r1, u32x4_t &k0,
-                                               u32x4_t &k1)
-{
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        k0[w] = (uint32_t)__builtin_amdgcn_update_dpp((int)r0[w], (int)r1[w], 0x128, 0xF, 0xC, false);
-        k1[w] = (uint32_t)__builtin_amdgcn_update_dpp((int)r1[w], (int)r0[w], 0x128, 0xF, 0x3, false);
-    }
-}
-
-__device__ __forceinline__ f32x4_t mfma16_f16(const u32x4_t &a, const u32x4_t &b, const f32x4_t &c)
-{
-    typedef _Float16 f16x8_t __attribute__((__vector_size__(8 * sizeof(_Float16))));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
 
 // Reducer workgroup r of a team: the team's steps k = r, r + R, ..., one
