@@ -593,7 +593,7 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
     // 10.3 / 10.7 / 12.0.  One slice of one or two strips gains nothing on
     // the split path (D = 64, T = 8192 16.0 / 27.3 / 15.0; D = 128 16.2 /
     // 31.8 / 15.9).
-    if (n == 4 && (D % 32) == 0 && D >= 192 && (D + 255) / 256 <= mhc::strip_max_slices() &&
+    if (n == 4 && D >= 192 && (D + 255) / 256 <= mhc::strip_max_slices() &&
         T < (int64_t{1} << 24)) {
         p.stripP = static_cast<int>((D + 255) / 256);
     }
@@ -717,7 +717,7 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
         // 21.4 / 19.0 / 29.1; D = 384, T = 4096 24.6 / 15.5 / 25.0; D = 192,
         // T = 8192 35.2 / 17.5 / 21.5) and stays the fallback of shapes the
         // rows path cannot hold.
-        if (p.stripP > 0) {
+        if (p.stripP > 0 && (D % 32) == 0) {
             // Single-slice teams (D = 256) included: the strip kernel also
             // beats the split path there (strip / split, us: T = 4096 11.8 /
             // 13.3, 8192 17.1 / 20.2, 32768 42.7 / 49.6).
@@ -759,6 +759,17 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
         }
     }
     const char *force = test_env("MHCPRE_FORCE_PATH");
+    // D % 32 == 16 (K % 128 != 0, the split path's shapes): the strip kernel in
+    // place of the split path's three, except narrow rows with many tokens.
+    // Measured on MI355X (bf16, gamma, executor launches, us, strip / split): D
+    // = 208: T = 64 11.1 / 12.2, 8192 20.1 / 18.6; D = 400: T = 777 11.7 / 11.8,
+    // 2048 13.0 / 11.9, 8192 22.7 / 24.0; D = 720: T = 777 12.5 / 11.7, 2048
+    // 16.2 / 14.7, 8192 28.2 / 32.6; D = 1200: T = 64 11.7 / 12.1, 777 13.1 /
+    // 14.0, 2048 16.9 / 18.8, 8192 37.3 / 44.2; D = 4880: T = 1 12.4 / 18.3, 777
+    // 20.3 / 30.1; D = 7056: T = 64 13.8 / 25.5, 8192 137.7 / 265.6.
+    const bool stripForced = force != nullptr && std::strcmp(force, "strip") == 0;
+    p.stripInstead = p.stripP > 0 && (D % 32) != 0 &&
+                     (stripForced || (force == nullptr && (D >= 960 || T <= 512 || (D >= 400 && T >= 8192))));
     // Slab kernel (n = 6), in place of the rows or split path's kernels.
     const bool slabForced = force != nullptr && std::strcmp(force, "slab") == 0;
     if (n == 6 && (slabForced || (force == nullptr && slab_faster(D, T))) &&
@@ -779,7 +790,7 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
             p.path = mhc::Path::kFused;
         } else if (std::strcmp(force, "rows") == 0 && p.rowsS > 0) {
             p.path = mhc::Path::kRows;
-        } else if (std::strcmp(force, "strip") == 0 && p.stripP > 0) {
+        } else if (std::strcmp(force, "strip") == 0 && p.stripP > 0 && (D % 32) == 0) {
             p.path = mhc::Path::kStrip;
         }
     }
@@ -869,6 +880,13 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
     default:
         p.wsTotal = splitEnd;
         break;
+    }
+    if (p.stripInstead) {
+        if (p.stripMaxTeams < 1 || (stripEnd > mhc::kScratchBytes && p.wsTotal <= mhc::kScratchBytes)) {
+            p.stripInstead = false;
+        } else {
+            p.wsTotal = std::max(p.wsTotal, stripEnd);
+        }
     }
     if (p.slab.P > 0) {
         const size_t slots = static_cast<size_t>(p.slab.groups) * p.slab.teams * mhc::slab_ring_slots();
@@ -1022,12 +1040,12 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     // error an earlier call of the process may have left there (the split
     // path makes no other HIP call before its first launch).
     (void)hipGetLastError();
-    if ((p.path != mhc::Path::kSplit || p.slab.P > 0) && !device_shape(device, shape)) {
+    if ((p.path != mhc::Path::kSplit || p.slab.P > 0 || p.stripInstead) && !device_shape(device, shape)) {
         return MHC_STATUS_HIP_ERROR;
     }
     const uint32_t launchId = next_launch_id();
     executor->lastLaunchId.store(launchId, std::memory_order_relaxed);
-    if (p.path == mhc::Path::kStrip) {
+    if (p.path == mhc::Path::kStrip || p.stripInstead) {
         // One workgroup per CU, all co-resident; each XCD's CUs hold at least
         // one team of stripP slice workgroups and one reducer workgroup.
         // Teams of two or more slices get at least two reducers: with one,
@@ -1115,6 +1133,9 @@ void prime_coresident(mhcPreExecutor *ex)
     void *scratch = nullptr;
     if (mhc::scratch_address(device, &scratch) != hipSuccess) {
         (void)hipGetLastError();
+    }
+    if (p.stripInstead) {
+        (void)cached_coresident(ex->stripCoresident, mhc::strip_max_coresident, p, shape.cus);
     }
     if (p.slab.P > 0) {
         (void)cached_coresident(ex->slabCoresident, mhc::slab_max_coresident, p, shape.cus);

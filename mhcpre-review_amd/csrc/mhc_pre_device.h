@@ -171,6 +171,8 @@ __device__ __forceinline__ f32x4_t mfma16(const u32x4_t &a, const u32x4_t &b, co
 constexpr int kCpolNt = 2;    // nontemporal: streamed once
 constexpr int kCpolDev = 16;  // sc1: device scope, written through, read past the L1 and L2 of another XCD
 
+constexpr int kPast = 0x40000000;  // an offset past every resource's end: reads zeros, stores nothing
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, int bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, bytes, 0x00020000);
@@ -367,6 +369,71 @@ __device__ __forceinline__ float ref_inv_rms(float sumsq, float invFlatDim, floa
     v = v + normEps;
     v = sqrtf(v);
     return 1.0f / v;
+}
+
+// The weights of a launch: phi [M][K] and gamma [K] or null, or the prepared
+// fragments.
+struct WeightsRef {
+    const float *phi;
+    const float *gamma;
+    const u32x4_t *bprep;
+    int K;
+};
+
+// Sums of one row over all of K, by one wave (every lane gets them): mix
+// columns j0 .. j0 + 7 (0 past M) and the sum of squares; rows past T read
+// zeros.  For work whose exchange wait expired: any wave can do it alone.
+template <int N, bool kBf16>
+__device__ __forceinline__ void own_sums(const WeightsRef &wt, const uint16_t *x, int64_t T, int64_t row, int j0,
+                                         float (&acc)[9])
+{
+    constexpr int M = Shape<N>::M;
+    constexpr int Q = M / 16;
+    const int K = wt.K;
+    const bool prep = wt.bprep != nullptr;
+    const bool hasGamma = wt.gamma != nullptr;
+    const __amdgpu_buffer_rsrc_t pr = make_rsrc(wt.phi, prep ? 0 : M * K * 4);
+    const __amdgpu_buffer_rsrc_t gr = make_rsrc(wt.gamma, hasGamma ? K * 4 : 0);
+    const __amdgpu_buffer_rsrc_t br = make_rsrc(wt.bprep, prep ? M * K * 4 : 0);
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x + (row < T ? row : 0) * K, row < T ? K * 2 : 0);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        acc[i] = 0.f;
+    }
+#pragma unroll 1
+    for (int k = (int)(threadIdx.x & 63); k < K; k += 64) {
+        const float xv = x_to_f32<kBf16>((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(xr, 2 * k, 0, 0));
+        const float gv = hasGamma ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gr, 4 * k, 0, 0)) : 1.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int j = j0 + i;
+            float b;
+            if (prep) {
+                // hi + lo of the prepared fragments' value (k, j): tiles j / 16
+                // and Q + j / 16, or (j >= 16 Q) lanes j % 16 and + 8 of tile 2Q.
+                const bool half = j >= 16 * Q;
+                const int tile = half ? 2 * Q : j >> 4;
+                const int f = (((k >> 5) * Shape<N>::NT + tile) * 64 + 16 * ((k >> 3) & 3) + (j & 15)) * 16 + 2 * (k & 7);
+                const int off = j < M ? f : kPast;
+                b = bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, off, 0, 0)) +
+                    bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
+                        br, off + (half ? 8 * 16 : Q * 64 * 16), 0, 0));
+            } else {
+                b = __uint_as_float(
+                        __builtin_amdgcn_raw_buffer_load_b32(pr, j < M ? (j * K + k) * 4 : kPast, 0, 0)) *
+                    gv;
+            }
+            acc[i] = __builtin_fmaf(xv, b, acc[i]);
+        }
+        acc[8] = __builtin_fmaf(xv, xv, acc[8]);
+    }
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) {
+            acc[i] = acc[i] + __shfl_xor(acc[i], m);
+        }
+    }
 }
 
 }  // namespace dev

@@ -88,11 +88,13 @@ struct Plan {
     int fusedTeams = 0;       // teams of fusedP workgroups
     int64_t fusedTiles = 0;   // 16-row tiles
 
-    // Strip path (n = 4, D % 32 == 0 from D = 192): P = ceil(D / 256) slice
+    // Strip path (n = 4, from D = 192): P = ceil(D / 256) slice
     // workgroups of 256 columns and R reducer workgroups per team, teams
     // formed inside one XCD or across the device.  stripR, stripXcds,
     // stripTeamsPerXcd and stripGrid are filled per launch from the device.
     int stripP = 0;
+    bool stripInstead = false;  // the strip kernel runs in place of the split path's (which stays
+                                // the fallback, its layout in the workspace)
     int stripMaxTeams = 0;  // teams the workspace's exchange rings are sized for (those of the
                             // device phase 1 planned for)
     int stripR = 0;

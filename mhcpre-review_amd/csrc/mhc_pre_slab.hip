@@ -98,7 +98,6 @@ constexpr int kRestBlocks = 3;             // blocks of 14 hPost / hRes columns
 constexpr int kRestCols = 14;
 constexpr int kMaxRest = 48;               // waves that take them
 static_assert(kRingSlots == kGroups * (kLag + 1) + kDoneLag, "ring slots");
-constexpr int kPast = 0x40000000;  // an offset past every resource's end: reads zeros, stores nothing
 constexpr int kXccIdReg = (3 << 11) | 20;  // s_getreg operand: HW_REG_XCC_ID, bits [3:0]
 
 template <int N>
@@ -167,6 +166,8 @@ __device__ __forceinline__ ArgsPtr phase_args()
     return p;
 }
 
+__device__ __forceinline__ WeightsRef weights_of(ArgsPtr p) { return {p->phi, p->gamma, p->bprep, (int)p->K}; }
+
 __device__ __forceinline__ uint32_t rec_tag(uint32_t pos, uint32_t epoch) { return (pos * 0x9E3779B1u) ^ epoch; }
 __device__ __forceinline__ uint32_t bcast_tag(uint32_t pos, uint32_t epoch)
 {
@@ -187,56 +188,6 @@ __device__ __forceinline__ void store_exchange(const u32x4_t &v, __amdgpu_buffer
         store16<0>(v, r, off);
     } else {
         store16<kCpolDev>(v, r, off);
-    }
-}
-
-// Sums of one row over all of K, by one wave (every lane gets them): mix
-// columns j0 .. j0 + 7 (0 past M) and the sum of squares.  Only for work whose
-// exchange wait expired.
-template <int N, bool kBf16>
-__device__ __forceinline__ void own_sums(ArgsPtr ap, int64_t row, int j0, float (&acc)[9])
-{
-    using Z = Geo<N>;
-    const int K = (int)ap->K;
-    const bool prep = ap->bprep != nullptr;
-    const bool hasGamma = ap->gamma != nullptr;
-    const __amdgpu_buffer_rsrc_t pr = make_rsrc(ap->phi, prep ? 0 : Z::M * K * 4);
-    const __amdgpu_buffer_rsrc_t gr = make_rsrc(ap->gamma, hasGamma ? K * 4 : 0);
-    const __amdgpu_buffer_rsrc_t br = make_rsrc(ap->bprep, prep ? Z::M * K * 4 : 0);
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(ap->x + (row < ap->T ? row : 0) * K, row < ap->T ? K * 2 : 0);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        acc[i] = 0.f;
-    }
-#pragma unroll 1
-    for (int k = (int)(threadIdx.x & 63); k < K; k += 64) {
-        const float xv = x_to_f32<kBf16>((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(xr, 2 * k, 0, 0));
-        const float gv = hasGamma ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gr, 4 * k, 0, 0)) : 1.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int j = j0 + i;
-            float b;
-            if (prep) {
-                // hi + lo of the prepared fragments' value (k, j).
-                const int f = (((k >> 5) * Z::NT + (j >> 4)) * 64 + 16 * ((k >> 3) & 3) + (j & 15)) * 16 + 2 * (k & 7);
-                const int off = j < Z::M ? f : kPast;
-                b = bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, off, 0, 0)) +
-                    bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, off + 1024 * Z::Q, 0, 0));
-            } else {
-                b = __uint_as_float(
-                        __builtin_amdgcn_raw_buffer_load_b32(pr, j < Z::M ? (j * K + k) * 4 : kPast, 0, 0)) *
-                    gv;
-            }
-            acc[i] = __builtin_fmaf(xv, b, acc[i]);
-        }
-        acc[8] = __builtin_fmaf(xv, xv, acc[8]);
-    }
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            acc[i] = acc[i] + __shfl_xor(acc[i], m);
-        }
     }
 }
 
@@ -372,7 +323,7 @@ __device__ __forceinline__ void crit_wave(ArgsPtr ap, const Team<N> &tm, int cls
 #pragma unroll 1
             for (int r = 0; r < 16; ++r) {
                 float own[9];
-                own_sums<N, kBf16>(ap, (int64_t)rt * 16 + r, 0, own);
+                own_sums<N, kBf16>(weights_of(ap), ap->x, ap->T, (int64_t)rt * 16 + r, 0, own);
                 if (rp == r >> 1) {
                     const float v = pick8(own, ic - 1);
                     acc.x = (r & 1) ? acc.x : v;
@@ -481,7 +432,7 @@ __device__ __forceinline__ void rest_wave(ArgsPtr ap, const Team<N> &tm, int ru,
 #pragma unroll 1
                 for (int h = 0; h < 2; ++h) {  // columns first .. + 7, then + 6 .. + 13
                     float own[9];
-                    own_sums<N, kBf16>(ap, (int64_t)rt * 16 + r, first + 6 * h, own);
+                    own_sums<N, kBf16>(weights_of(ap), ap->x, ap->T, (int64_t)rt * 16 + r, first + 6 * h, own);
                     const int i = lane % kRestCols - 6 * h;
                     const float v = pick8(own, i & 7);
                     const bool mine = quad == r >> 2 && i >= 0 && i < 8;
@@ -1035,7 +986,7 @@ __global__ __launch_bounds__(kThreads) void slab_kernel(SlabArgs a)
                 break;
             }
             float own[9];
-            own_sums<N, kBf16>(ca, row, 0, own);
+            own_sums<N, kBf16>(weights_of(ca), ca->x, ca->T, row, 0, own);
             const float ir = ref_inv_rms(own[8], ca->invFlatDim, ca->normEps);
             const int c = col0 + lane;
             float v = 0.f;

@@ -1,4 +1,4 @@
-// Strip kernel for gfx950 (n = 4, D % 32 == 0): x is read from HBM once,
+// Strip kernel for gfx950 (n = 4, D % 16 == 0): x is read from HBM once,
 // held in VGPRs in a ring of row tiles until its hIn is written, and the
 // cross-workgroup exchange of the K-reduction runs in the shadow of the x
 // stream.
@@ -286,7 +286,7 @@ struct ColPoll {
     }
 };
 
-template <int N, int MaxS>
+template <int N, int MaxS, bool kBf16, bool kOwn>
 __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int ntiles, int r, int R,
                                            bool local, float *lds, uint32_t prevEpoch,
                                            uint32_t *epochSh)
@@ -325,6 +325,42 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
     const float bias1 = a.bias[p1.c < N ? p1.c : 0];
     const float bias2 = a.bias[p2.c - 1];
     bool timedOut = false;
+    // kOwn: the sums of mix columns j0 .. j1 - 1 (and, with j0 = 0, the sum of
+    // squares) of a tile whose records did not come, into group 0 of `sums`
+    // (the others zero), a wave per row.
+    const auto own_phase = [&](int rt, int j0, int j1) {
+        const int items = j0 == 0 ? Poll1::ITEMS : Poll2::ITEMS;
+        const int groups = j0 == 0 ? Poll1::SG : Poll2::SG;
+        __syncthreads();
+        for (int i = tid; i < 2 * groups * items; i += kWaves * 64) {
+            sums[i] = 0.f;
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int row = tid >> 6; row < 16; row += kWaves) {
+#pragma unroll 1
+            for (int j = j0; j < j1; j += 8) {
+                float own[9];
+                own_sums<N, kBf16>(WeightsRef{a.phi, a.gamma, a.bprep, (int)a.K}, a.x, a.T, (int64_t)rt * 16 + row, j,
+                                   own);
+                // Item (column j - j0) * 8 + row / 2 of the phase, component
+                // row % 2; the sum of squares is phase 1's last column.
+                const int at = 2 * (row >> 1) + (row & 1);
+                if ((tid & 63) == 0) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        if (j + i < j1) {
+                            sums[16 * (j + i - j0) + at] = own[i];
+                        }
+                    }
+                    if (j0 == 0) {
+                        sums[16 * N + at] = own[8];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    };
     for (int k = r; k < ntiles; k += R) {
         const int rt = team + a.numTeams * k;
         const uint32_t slot = (uint32_t)(team * kRingSlots + k % kRingSlots);
@@ -347,7 +383,9 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
                 break;  // an earlier wait expired: no more waiting in this launch
             }
             if (spins >= a.spinLimit) {
-                record_timeout(a, tid);
+                if constexpr (!kOwn) {
+                    record_timeout(a, tid);
+                }
                 timedOut = true;
                 break;
             }
@@ -361,6 +399,11 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
             sums[(p1.sg * Poll1::ITEMS + tid % Poll1::ITEMS) * 2 + 1] = acc.y;
         }
         lds_barrier();
+        if constexpr (kOwn) {
+            if (!got) {
+                own_phase(rt, 0, N);
+            }
+        }
         // Wave 0 finishes phase 1 (its lanes 0 .. 8(N+1)-1 are the items):
         // the groups' sums in order, invRms in the lanes of column N (lane
         // 8N + i has rows 2i, 2i + 1), handed to the hPre lanes of the same
@@ -428,7 +471,9 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
                 break;
             }
             if (spins >= a.spinLimit) {
-                record_timeout(a, tid);
+                if constexpr (!kOwn) {
+                    record_timeout(a, tid);
+                }
                 timedOut = true;
                 break;
             }
@@ -442,6 +487,11 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
             sums[(p2.sg * Poll2::ITEMS + tid % Poll2::ITEMS) * 2 + 1] = acc.y;
         }
         lds_barrier();
+        if constexpr (kOwn) {
+            if (!got) {
+                own_phase(rt, N, COLS - 1);
+            }
+        }
         if (tid < Poll2::ITEMS) {
             float2 gs[Poll2::SG];
 #pragma unroll
@@ -476,7 +526,12 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
     }
 }
 
-template <int N, bool kBf16, bool kPrep>
+// kOwn (D % 32 == 16): these widths ran kernels that wait for nobody before, so
+// a workgroup whose wait expires computes what it waited for itself, from x
+// and the weights, instead of writing NaN and reporting it.  One launch in
+// place of three: D = 1200, T = 777 14.9 -> 12.5 us as an eager operator call,
+// D = 7056, T = 8192 266 -> 138 us.
+template <int N, bool kBf16, bool kPrep, bool kOwn>
 __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
 {
     using S = Shape<N>;
@@ -544,13 +599,13 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
         float *lds = &part[0][0][0][0];
         const int rr = role - a.P;
         if (a.P <= 8) {
-            reducer_wg<N, 8>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, 8, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
         } else if (a.P <= 16) {
-            reducer_wg<N, 16>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, 16, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
         } else if (a.P <= 32) {
-            reducer_wg<N, 32>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, 32, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
         } else {
-            reducer_wg<N, kMaxSlices>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, kMaxSlices, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
         }
         return;
     }
@@ -663,11 +718,15 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
 #pragma unroll
         for (int i = 0; i < KW; ++i) {
             const int ks = half + kGroups * i;
-            const int64_t gks = ((int64_t)(ks >> 1) * a.D + col0 + 32 * (ks & 1)) / 32;
-            const bool ksLive = col0 + 32 * (ks & 1) < Di;  // the k-step's 32 columns are within D
+            // (D % 32 == 16: a stream's k-steps may begin inside a prepared one;
+            // each lane then takes its 8 values of k from where they are)
+            const int dc = col0 + 32 * (ks & 1) + (kOwn ? 8 * grp : 0);
+            const int64_t k0 = (int64_t)(ks >> 1) * a.D + dc;
+            const int from = kOwn ? 16 * (int)((k0 >> 3) & 3) + rl : lane;
+            const bool ksLive = dc < Di;  // the k-step's columns are within D
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                pf[i][t] = ksLive ? a.bprep[(gks * NT + t) * 64 + lane] : u32x4_t{0u, 0u, 0u, 0u};
+                pf[i][t] = ksLive ? a.bprep[((k0 >> 5) * NT + t) * 64 + from] : u32x4_t{0u, 0u, 0u, 0u};
             }
         }
     } else {
@@ -827,6 +886,7 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     // Exchange ring slot of own step jj (team step G jj + group).
     auto slot_of = [&](int jj) { return teamI * kRingSlots + (kGroups * jj + half) % kRingSlots; };
     bool timedOut = false;
+    int failFrom = 0;  // kOwn: the own tile whose wait expired first
 
     // Meeting count of the other group once it has run all its steps (the
     // meetings are in the steps with a tile, own steps 0 .. nmine - 1).
@@ -867,7 +927,9 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
                     break;
                 }
                 if (spins >= spinLimit) {
-                    if (lane == 0) {
+                    if constexpr (kOwn) {
+                        failFrom = jh;
+                    } else if (lane == 0) {
                         st_status(statusW, launchId);
                     }
                     timedOut = true;
@@ -918,7 +980,8 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
                               bcastAll, (slot_of(jpc) * RC::BWORDS + lane) * 8, 0, kCpolDev));
         }
         {
-            const __amdgpu_buffer_rsrc_t hr = make_rsrc(h_tile(jh), liveH && stripLive ? rows_of(jh) * Di * 2 : 0);
+            const __amdgpu_buffer_rsrc_t hr = make_rsrc(
+                h_tile(jh), liveH && stripLive && !(kOwn && timedOut) ? rows_of(jh) * Di * 2 : 0);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 store16<kCpolNt>(hout[h], hr, hLane + 8 * h * Di * 2);
@@ -1116,34 +1179,60 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
         }
     });
     // A wave whose wait expired also marks the caller's status word, once,
-    // outside the loop.
-    if (timedOut && lane == 0) {
+    // outside the loop (kOwn: it computes its hIn from that tile on, alone).
+    if constexpr (kOwn) {
+        if (timedOut) {
+#pragma unroll 1
+            for (int i = 16 * failFrom; i < 16 * nmine; ++i) {
+                const int64_t row = (int64_t)tile_of(i >> 4) * 16 + (i & 15);
+                if (row >= T32) {
+                    break;
+                }
+                float own[9];
+                own_sums<N, kBf16>(WeightsRef{a.phi, a.gamma, a.bprep, Ki}, a.x, a.T, row, 0, own);
+                const float ir = ref_inv_rms(own[8], a.invFlatDim, a.normEps);
+                const int c = col0 + lane;
+                float v = 0.f;
+#pragma unroll
+                for (int s = 0; s < N; ++s) {
+                    const float pre = ref_sigmoid(own[s] * (ir * a.alpha[0]), a.bias[s], a.hcEps);
+                    if (c < Di) {
+                        const float prod = pre * x_to_f32<kBf16>(a.x[row * Ki + s * Di + c]);
+                        v = s == 0 ? prod : v + prod;
+                    }
+                }
+                if (c < Di) {
+                    a.hIn[row * Di + c] = (uint16_t)f32_to_x<kBf16>(v);
+                }
+            }
+        }
+    } else if (timedOut && lane == 0) {
         st_status_word(a.statusWord);
     }
     // Workgroup 0 (always a slice workgroup of team 0) advances the
     // workspace's epoch once every workgroup has taken this one.
     if (g == 0 && w == 0) {
         if (!epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, spinLimit) &&
-            lane == 0) {
+            !kOwn && lane == 0) {
             st_status(statusW, launchId);
             st_status_word(a.statusWord);
         }
     }
 }
 
-template <int N, bool kBf16, bool kPrep>
+template <int N, bool kBf16, bool kPrep, bool kOwn>
 int strip_coresident_t(int numCUs)
 {
     int perCU = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &perCU, reinterpret_cast<const void *>(&strip_kernel<N, kBf16, kPrep>), kWaves * 64, 0) !=
+            &perCU, reinterpret_cast<const void *>(&strip_kernel<N, kBf16, kPrep, kOwn>), kWaves * 64, 0) !=
         hipSuccess) {
         return -1;
     }
     return perCU * numCUs;
 }
 
-template <int N, bool kBf16, bool kPrep>
+template <int N, bool kBf16, bool kPrep, bool kOwn>
 hipError_t launch_strip_t(const Plan &p, void *workspace, uint32_t launchId, hipStream_t stream)
 {
     char *ws = static_cast<char *>(workspace);
@@ -1177,18 +1266,33 @@ hipError_t launch_strip_t(const Plan &p, void *workspace, uint32_t launchId, hip
     a.launchId = launchId;
     a.spinLimit = p.spinLimit;
     if (!p.fusedCooperative) {
-        hipLaunchKernelGGL((strip_kernel<N, kBf16, kPrep>), dim3((unsigned)p.stripGrid), dim3(kWaves * 64), 0,
+        hipLaunchKernelGGL((strip_kernel<N, kBf16, kPrep, kOwn>), dim3((unsigned)p.stripGrid), dim3(kWaves * 64), 0,
                            stream, a);
         return hipGetLastError();
     }
     // Cooperative launch (MHCPRE_LAUNCH=cooperative): co-residency of the
     // whole grid is guaranteed even next to concurrent work.
     void *args[] = {&a};
-    return hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&strip_kernel<N, kBf16, kPrep>),
+    return hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&strip_kernel<N, kBf16, kPrep, kOwn>),
                                       dim3((unsigned)p.stripGrid), dim3(kWaves * 64), args, 0,
                                       stream);
 }
 
+}  // namespace
+
+namespace {
+// Calls f with the flags of the instance a plan takes.
+template <typename F>
+auto strip_instance(const Plan &p, F &&f)
+{
+    const auto own = [&](auto bf16, auto prep) {
+        return p.D % 32 != 0 ? f(bf16, prep, std::true_type{}) : f(bf16, prep, std::false_type{});
+    };
+    const auto prep = [&](auto bf16) {
+        return p.bprep != nullptr ? own(bf16, std::true_type{}) : own(bf16, std::false_type{});
+    };
+    return p.isBf16 ? prep(std::true_type{}) : prep(std::false_type{});
+}
 }  // namespace
 
 hipError_t launch_strip(const Plan &p, void *workspace, uint32_t launchId, hipStream_t stream)
@@ -1196,12 +1300,10 @@ hipError_t launch_strip(const Plan &p, void *workspace, uint32_t launchId, hipSt
     if (p.n != 4) {
         return hipErrorNotSupported;
     }
-    if (p.bprep != nullptr) {
-        return p.isBf16 ? launch_strip_t<4, true, true>(p, workspace, launchId, stream)
-                        : launch_strip_t<4, false, true>(p, workspace, launchId, stream);
-    }
-    return p.isBf16 ? launch_strip_t<4, true, false>(p, workspace, launchId, stream)
-                    : launch_strip_t<4, false, false>(p, workspace, launchId, stream);
+    return strip_instance(p, [&](auto bf16, auto prep, auto own) {
+        return launch_strip_t<4, decltype(bf16)::value, decltype(prep)::value, decltype(own)::value>(p, workspace,
+                                                                                                    launchId, stream);
+    });
 }
 
 int strip_ring_slots() { return kRingSlots; }
@@ -1233,12 +1335,9 @@ int strip_max_coresident(const Plan &p, int numCUs)
     if (p.n != 4) {
         return -1;
     }
-    if (p.bprep != nullptr) {
-        return p.isBf16 ? strip_coresident_t<4, true, true>(numCUs)
-                        : strip_coresident_t<4, false, true>(numCUs);
-    }
-    return p.isBf16 ? strip_coresident_t<4, true, false>(numCUs)
-                    : strip_coresident_t<4, false, false>(numCUs);
+    return strip_instance(p, [&](auto bf16, auto prep, auto own) {
+        return strip_coresident_t<4, decltype(bf16)::value, decltype(prep)::value, decltype(own)::value>(numCUs);
+    });
 }
 
 }  // namespace mhc
