@@ -104,7 +104,8 @@ typedef struct mhcPreExecutor mhcPreExecutor;
  * the team count is that of the device holding x (of MI355X when the runtime
  * cannot tell).  The two-pass paths hold partial sums that grow with T.  A
  * shape that runs the slab kernel asks for the larger of its exchange rings
- * (which do not grow with T) and its path's own layout.
+ * (which do not grow with T) and its path's own layout, and one that runs the
+ * cell kernel for the larger of its records (at most 2.3 MB) and that layout.
  */
 MHC_API int mhcPreGetWorkspaceSize(const mhcTensor *x, const mhcTensor *phi, const mhcTensor *alpha,
                            const mhcTensor *bias, const mhcTensor *gamma, float normEps,
@@ -147,9 +148,10 @@ MHC_API int mhcPreGetWorkspaceSizeWithHPre(const mhcTensor *x, const mhcTensor *
  * uses a cooperative launch, which guarantees co-residency next to concurrent
  * work but dispatches more slowly (about 20 us per launch on MI355X).
  *
- * The slab kernel (n = 6) waits between workgroups in the same way, but a
- * workgroup whose wait expires computes what it waited for itself: such a
- * launch is slow and its outputs are right, so nothing is reported.
+ * The cell kernel (small batches), the slab kernel (n = 6) and the strip kernel
+ * at D % 32 == 16 wait between workgroups in the same way, but a workgroup whose
+ * wait expires computes what it waited for itself: such a launch is slow and
+ * its outputs are right, so nothing is reported.
  *
  * A launch may be captured into a HIP graph and replayed: the exchange epoch
  * that tells the current launch's data from stale workspace contents is kept
@@ -263,8 +265,9 @@ MHC_API const char *mhcPreStatusString(int status);
 
 /* Which kernel path an executor launches (diagnostics and benchmarks):
  * writes a static NUL-terminated name to *name.  The name is that of the
- * path the shape belongs to: "rows" and "split" shapes with n = 6 run the slab
- * kernel instead of the path's own kernels where it is faster. */
+ * path the shape belongs to: small batches run the cell kernel, "rows" and
+ * "split" shapes with n = 6 the slab kernel, and "split" shapes with n = 4 the
+ * strip kernel, instead of the path's own kernels where that is faster. */
 MHC_API int mhcPreExecutorPath(const mhcPreExecutor *executor, const char **name);
 
 /*

@@ -92,6 +92,7 @@ struct mhcPreExecutor {
     std::atomic<int> stripCoresident{-2};
     std::atomic<int> fusedCoresident{-2};
     std::atomic<int> slabCoresident{-2};
+    std::atomic<int> cellCoresident{-2};
     // The caller's sticky device status word (mhcPreExecutorSetStatusWord),
     // or null.
     std::atomic<uint32_t *> statusWord{nullptr};
@@ -278,6 +279,61 @@ mhc::SlabGeometry slab_geometry(int64_t D, int64_t T, const DeviceShape &s)
     }
     return best;
 }
+
+// Workgroups of the cell kernel with slices of 64 `strips` columns; 0: more
+// than its exchange and its launch are made for.
+int64_t cell_grid(int n, int64_t D, int64_t T, int strips)
+{
+    const int64_t P = (D + 64 * strips - 1) / (64 * strips);
+    const int64_t tiles = (T + 15) / 16;
+    const int64_t grid = P * tiles * ((n * n + 2 * n + 15) / 16);
+    return P <= 64 && tiles <= 1024 && grid <= 1024 ? grid : 0;
+}
+
+// Slice width of the cell kernel, and whether it is faster than the kernels of
+// the shape's path.
+//
+// Narrow slices (one strip) spread the weights over twice the CUs while those
+// are there to take them, wide ones halve the records that every workgroup
+// reads.  Measured on MI355X (bf16, gamma, in a graph, us, one strip / two): n =
+// 4: D = 256, T = 16 5.4 / 6.0, T = 256 5.7 / 6.0, T = 512 6.5 / 6.1; D = 1024,
+// T = 64 6.3 / 6.4, T = 128 7.5 / 7.0; D = 2560, T = 32 6.9 / 6.8; n = 6: D =
+// 1024, T = 64 7.1 / 7.5, T = 96 8.4 / 8.2; D = 2560, T = 16 7.0 / 7.4, T = 32
+// 7.9 / 7.7; n = 8: D = 512, T = 128 8.4 / 8.9; D = 2560, T = 16 8.1 / 9.1, T =
+// 32 10.4 / 10.3.
+//
+// Against the path's kernels it wins while the device holds one workgroup per
+// CU and, where few slices exchange records, two.  Measured as above (us, cell /
+// path; a launch less saves the host about 3 us besides): n = 4: D = 256, T =
+// 16 5.4 / 6.5, T = 1024 6.8 / 10.7; D = 784, T = 16 6.1 / 12.0, T = 512 9.1 /
+// 11.9; D = 1024, T = 512 8.7 / 10.8; D = 2560, T = 128 8.4 / 9.5; D = 4096, T =
+// 64 7.8 / 8.8, T = 96 9.3 / 9.1; D = 7168, T = 16 7.4 / 8.6, T = 32 8.1 / 8.7,
+// T = 64 9.4 / 9.0; n = 6: D = 512, T = 512 9.5 / 12.2; D = 2560, T = 16 7.0 /
+// 9.1, T = 128 10.1 / 11.4; D = 4096, T = 32 8.4 / 9.4, T = 48 10.5 / 9.6; D =
+// 7168, T = 16 9.0 / 9.5, T = 32 11.7 / 9.6; n = 8: D = 256, T = 512 10.4 /
+// 12.6; D = 1024, T = 16 6.7 / 10.4, T = 128 11.2 / 12.0; D = 2560, T = 32 10.3
+// / 10.8, T = 48 11.0 / 11.0; D = 4096, T = 16 9.6 / 10.7, T = 32 12.4 / 11.0;
+// D = 7168, T = 16 13.4 / 11.5.
+struct CellShape {
+    int strips = 1;
+    bool faster = false;
+};
+CellShape cell_shape(int n, int64_t D, int64_t T)
+{
+    CellShape c;
+    const int64_t P1 = (D + 63) / 64;
+    const int64_t P2 = (D + 127) / 128;
+    const int64_t tiles = (T + 15) / 16;
+    c.strips = tiles * P1 <= 64 && P1 <= (n == 4 ? 16 : 40) ? 1 : 2;
+    if (const char *forced = test_env("MHCPRE_CELL")) {
+        c.strips = std::atoi(forced) == 1 ? 1 : 2;
+    }
+    const int64_t columnTiles = (n * n + 2 * n + 15) / 16;
+    const int64_t grid = cell_grid(n, D, T, 2);
+    c.faster = c.strips == 1 || (grid > 0 && grid <= (P2 * columnTiles <= 64 ? 512 : 256));
+    return c;
+}
+
 
 // Where the slab kernel is faster than the kernels of its shape's path (n = 6).
 // Measured on MI355X (bf16, gamma, back to back, us, slab / the rows or split
@@ -759,6 +815,17 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
         }
     }
     const char *force = test_env("MHCPRE_FORCE_PATH");
+    // Cell kernel (small batches), in place of the path's kernels.
+    const bool cellForced = force != nullptr && std::strcmp(force, "cell") == 0;
+    if (cellForced || force == nullptr) {
+        const CellShape c = cell_shape(n, D, T);
+        const int64_t grid = cell_grid(n, D, T, c.strips);
+        if (cellForced ? grid > 0 : c.faster) {
+            p.cellStrips = c.strips;
+            p.cellP = static_cast<int>((D + 64 * c.strips - 1) / (64 * c.strips));
+            p.cellGrid = static_cast<int>(grid);
+        }
+    }
     // D % 32 == 16 (K % 128 != 0, the split path's shapes): the strip kernel in
     // place of the split path's three, except narrow rows with many tokens.
     // Measured on MI355X (bf16, gamma, executor launches, us, strip / split): D
@@ -768,11 +835,11 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
     // 14.0, 2048 16.9 / 18.8, 8192 37.3 / 44.2; D = 4880: T = 1 12.4 / 18.3, 777
     // 20.3 / 30.1; D = 7056: T = 64 13.8 / 25.5, 8192 137.7 / 265.6.
     const bool stripForced = force != nullptr && std::strcmp(force, "strip") == 0;
-    p.stripInstead = p.stripP > 0 && (D % 32) != 0 &&
+    p.stripInstead = p.cellP == 0 && p.stripP > 0 && (D % 32) != 0 &&
                      (stripForced || (force == nullptr && (D >= 960 || T <= 512 || (D >= 400 && T >= 8192))));
     // Slab kernel (n = 6), in place of the rows or split path's kernels.
     const bool slabForced = force != nullptr && std::strcmp(force, "slab") == 0;
-    if (n == 6 && (slabForced || (force == nullptr && slab_faster(D, T))) &&
+    if (n == 6 && p.cellP == 0 && (slabForced || (force == nullptr && slab_faster(D, T))) &&
         D <= mhc::slab_max_slices() * mhc::slab_columns() && T < (int64_t{1} << 24)) {
         DeviceShape shape = kPlanShapeDefault;
         if (planDevice < 0 || !device_shape_of(planDevice, shape)) {
@@ -880,6 +947,12 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
     default:
         p.wsTotal = splitEnd;
         break;
+    }
+    if (p.cellP > 0) {
+        p.wsCellRecs = mhc::kWsHeaderBytes;
+        p.wsTotal = std::max(p.wsTotal, p.wsCellRecs + align_up(static_cast<size_t>(p.cellGrid) *
+                                                                    mhc::cell_record_bytes(),
+                                                                256));
     }
     if (p.stripInstead) {
         if (p.stripMaxTeams < 1 || (stripEnd > mhc::kScratchBytes && p.wsTotal <= mhc::kScratchBytes)) {
@@ -994,11 +1067,11 @@ int cached_coresident(std::atomic<int> &slot, int (*query)(const mhc::Plan &, in
         (void)hipGetLastError();
         return query(p, cus);
     }
-    using Key = std::tuple<uintptr_t, int, int, bool, bool, int, int>;
+    using Key = std::tuple<uintptr_t, int, int, bool, bool, int, int, int>;
     static std::mutex mu;
     static std::map<Key, int> known;
     const Key key{reinterpret_cast<uintptr_t>(query), device, p.n, p.isBf16, p.bprep != nullptr,
-                  p.fusedDw, cus};
+                  p.fusedDw, p.cellStrips, cus};
     {
         std::lock_guard<std::mutex> lock(mu);
         const auto it = known.find(key);
@@ -1040,12 +1113,17 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     // error an earlier call of the process may have left there (the split
     // path makes no other HIP call before its first launch).
     (void)hipGetLastError();
-    if ((p.path != mhc::Path::kSplit || p.slab.P > 0 || p.stripInstead) && !device_shape(device, shape)) {
+    if ((p.path != mhc::Path::kSplit || p.slab.P > 0 || p.stripInstead || p.cellP > 0) && !device_shape(device, shape)) {
         return MHC_STATUS_HIP_ERROR;
     }
     const uint32_t launchId = next_launch_id();
     executor->lastLaunchId.store(launchId, std::memory_order_relaxed);
-    if (p.path == mhc::Path::kStrip || p.stripInstead) {
+    if (p.cellP > 0 && p.cellGrid <= mhc::kMaxEpochGrid &&
+        cached_coresident(executor->cellCoresident, mhc::cell_max_coresident, p, shape.cus) >= p.cellGrid) {
+        err = mhc::launch_cell(p, workspace, stream);
+        done = true;
+    }
+    if (!done && (p.path == mhc::Path::kStrip || p.stripInstead)) {
         // One workgroup per CU, all co-resident; each XCD's CUs hold at least
         // one team of stripP slice workgroups and one reducer workgroup.
         // Teams of two or more slices get at least two reducers: with one,
@@ -1133,6 +1211,9 @@ void prime_coresident(mhcPreExecutor *ex)
     void *scratch = nullptr;
     if (mhc::scratch_address(device, &scratch) != hipSuccess) {
         (void)hipGetLastError();
+    }
+    if (p.cellP > 0) {
+        (void)cached_coresident(ex->cellCoresident, mhc::cell_max_coresident, p, shape.cus);
     }
     if (p.stripInstead) {
         (void)cached_coresident(ex->stripCoresident, mhc::strip_max_coresident, p, shape.cus);

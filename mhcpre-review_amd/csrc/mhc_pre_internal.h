@@ -107,6 +107,12 @@ struct Plan {
     // (the fallback on a device that cannot co-schedule its grid).
     SlabGeometry slab;
 
+    // Cell kernel (small batches; cellP == 0: not taken): one launch that runs
+    // in place of the path's own kernels, which stay the fallback.
+    int cellP = 0;       // slices of 64 cellStrips columns
+    int cellStrips = 1;  // 1 or 2
+    int cellGrid = 0;    // workgroups: cellP per 16-row and 16-column tile
+
     // Rows path (K % 128 == 0): rowsS K-ranges (contiguous runs of
     // rows_stage_ksteps()-k-step stages) over rowsBlocks blocks of
     // rows_block_rows() rows.
@@ -139,6 +145,7 @@ struct Plan {
     size_t wsSlabFlags = 0;   // slab: per-team rings of the slices' flags
     size_t wsSlabDone = 0;    // slab: the reducer waves' done words
     size_t wsSlabRecs = 0;    // slab: per-team rings of P exchange records
+    size_t wsCellRecs = 0;    // cell: [tile][cellP] records
     size_t wsTotal = 0;
 
     // Bound device pointers (caller memory).
@@ -171,6 +178,11 @@ hipError_t launch_split(const Plan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_fused(const Plan &plan, void *workspace, uint32_t launchId, hipStream_t stream);
 
 hipError_t launch_strip(const Plan &plan, void *workspace, uint32_t launchId, hipStream_t stream);
+
+// Cell kernel (mhc_pre_cell.hip).
+hipError_t launch_cell(const Plan &plan, void *workspace, hipStream_t stream);
+int cell_max_coresident(const Plan &plan, int numCUs);
+size_t cell_record_bytes();
 
 // Slab kernel (mhc_pre_slab.hip): one launch, x read once.
 hipError_t launch_slab(const Plan &plan, void *workspace, hipStream_t stream);

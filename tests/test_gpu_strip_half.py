@@ -40,17 +40,21 @@ def test_strip_at_half_step_widths(pkg, orc, device, T, D, is_bf16, has_gamma, p
     x, phi, alpha, bias, gamma = _inputs(T, D, is_bf16, has_gamma)
     _say(f"[strip half] T={T} D={D} bf16={is_bf16} gamma={has_gamma} prepared={prepared}")
     ref = orc.mhc_pre(x, is_bf16, phi, alpha, bias, gamma)
-    plain = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma)
+    plain = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="strip")
+    os.environ["MHCPRE_FORCE_PATH"] = "strip"
+    try:
+        xt, pt, at, bt, gt = to_device(pkg, device, x, is_bf16, phi, alpha, bias, gamma)
+        op = pkg.MhcPreOp(xt, None, at, bt, None, h_pre=True, weights=pkg.MhcPreWeights(pt, gt, N))
+    finally:
+        os.environ.pop("MHCPRE_FORCE_PATH", None)
     assert plain.pop("path") == "split"
     check(plain, ref, x, is_bf16, orc)
     if prepared:  # the same bits from prepared weights
-        xt, pt, at, bt, gt = to_device(pkg, device, x, is_bf16, phi, alpha, bias, gamma)
-        op = pkg.MhcPreOp(xt, None, at, bt, None, h_pre=True, weights=pkg.MhcPreWeights(pt, gt, N))
         op.launch(check=True)
         got = fetch(op)
         for k in plain:
             assert np.array_equal(got[k], plain[k]), k
-        op.close()
+    op.close()
 
 
 @pytest.mark.parametrize("T,D,prepared", [(300, 1200, False), (200, 720, True)])
@@ -63,10 +67,12 @@ def test_expired_waits_are_computed(pkg, orc, device, T, D, prepared):
     weights = pkg.MhcPreWeights(pt, gt, N) if prepared else None
     args = (xt, None, at, bt, None) if prepared else (xt, pt, at, bt, gt)
     os.environ["MHCPRE_SPIN_LIMIT"] = "0"
+    os.environ["MHCPRE_FORCE_PATH"] = "strip"
     try:
         op = pkg.MhcPreOp(*args, h_pre=True, weights=weights)
     finally:
         os.environ.pop("MHCPRE_SPIN_LIMIT", None)
+        os.environ.pop("MHCPRE_FORCE_PATH", None)
     ref = orc.mhc_pre(x, True, phi, alpha, bias, gamma)
     for _ in range(2):
         for t in op.outputs():
