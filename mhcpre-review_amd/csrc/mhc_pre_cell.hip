@@ -451,7 +451,7 @@ __global__ __launch_bounds__((Cell<N, NS>::kThreads), (Cell<N, NS>::kWavesPerSim
     // Workgroup 0 advances the workspace's epoch once every workgroup has
     // taken this one; its last wave (which has no part in hIn) waits for that.
     if (group == 0 && p == 0 && w == W - 1) {
-        (void)epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, P * (int)(gridDim.y * gridDim.z), a.spinLimit);
+        (void)epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, P * (int)(gridDim.y * gridDim.z), kPublishPolls);
     }
 }
 
@@ -490,7 +490,7 @@ struct Instance {
         a.normEps = p.normEps;
         a.hcEps = p.hcEps;
         a.invFlatDim = p.invFlatDim;
-        a.spinLimit = p.spinLimit;
+        a.spinLimit = p.cellSpinLimit();
         const unsigned tiles = (unsigned)((p.T + 15) / 16);
         const dim3 grid((unsigned)p.cellP, tiles, (unsigned)(p.cellGrid / (p.cellP * tiles)));
         const dim3 block(Cell<N, NS>::kThreads);

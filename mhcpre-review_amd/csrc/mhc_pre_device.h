@@ -302,6 +302,10 @@ __device__ __forceinline__ void epoch_mark(void *ws, size_t seenOff, uint32_t ep
                                           16 /* sc1 */);
 }
 
+// epoch_publish's limit in kernels whose other waits are shorter (about a
+// second): their late workgroups must not read the advanced epoch.
+constexpr uint32_t kPublishPolls = 1u << 20;
+
 // One whole wave: waits (bounded by spinLimit polls) until the slots of all
 // `grid` workgroups hold `epoch`, then stores it as the header's epoch.
 // Returns false if the wait expired (the epoch is stored anyway, so that the

@@ -72,6 +72,13 @@ struct Plan {
     // gives up (about a second).  MHCPRE_SPIN_LIMIT at phase 1 overrides it,
     // for tests of the timeout path.
     uint32_t spinLimit = 1u << 20;
+    // The same for kernels whose expired waits are computed instead: about as
+    // long as the computation takes, so that two such launches that hold half
+    // of each other's CUs do not stand still for a second (the cell kernel
+    // recomputes a row tile in up to 0.2 ms, the slab kernel and the strip
+    // kernel at D % 32 == 16 a workgroup's rows in some 20 ms).
+    uint32_t cellSpinLimit() const { return spinLimit < (1u << 9) ? spinLimit : 1u << 9; }
+    uint32_t ownSpinLimit() const { return spinLimit < (1u << 14) ? spinLimit : 1u << 14; }
     float normEps = 1e-6f;
     float hcEps = 1e-6f;
     float invFlatDim = 0.f;  // fl(1.0f / K), as code/op_host/mhc_pre.cpp:154

@@ -1007,7 +1007,7 @@ __global__ __launch_bounds__(kThreads) void slab_kernel(SlabArgs a)
     // every workgroup has taken this one.
     if (g == 0 && w == 0) {
         const ArgsPtr ea = phase_args();
-        (void)epoch_publish(ea->hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, ea->spinLimit);
+        (void)epoch_publish(ea->hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, kPublishPolls);
     }
 }
 
@@ -1056,7 +1056,7 @@ hipError_t launch_slab_t(const Plan &p, void *workspace, hipStream_t stream)
     a.normEps = p.normEps;
     a.hcEps = p.hcEps;
     a.invFlatDim = p.invFlatDim;
-    a.spinLimit = p.spinLimit;
+    a.spinLimit = p.ownSpinLimit();
     if (!p.fusedCooperative) {
         hipLaunchKernelGGL((slab_kernel<N, kBf16, kPrep>), dim3((unsigned)p.slab.grid), dim3(kThreads), 0,
                            stream, a);

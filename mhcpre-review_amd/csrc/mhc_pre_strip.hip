@@ -1212,7 +1212,7 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     // Workgroup 0 (always a slice workgroup of team 0) advances the
     // workspace's epoch once every workgroup has taken this one.
     if (g == 0 && w == 0) {
-        if (!epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, spinLimit) &&
+        if (!epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, kOwn ? kPublishPolls : spinLimit) &&
             !kOwn && lane == 0) {
             st_status(statusW, launchId);
             st_status_word(a.statusWord);
@@ -1264,7 +1264,7 @@ hipError_t launch_strip_t(const Plan &p, void *workspace, uint32_t launchId, hip
     a.hcEps = p.hcEps;
     a.invFlatDim = p.invFlatDim;
     a.launchId = launchId;
-    a.spinLimit = p.spinLimit;
+    a.spinLimit = (p.D % 32) != 0 ? p.ownSpinLimit() : p.spinLimit;
     if (!p.fusedCooperative) {
         hipLaunchKernelGGL((strip_kernel<N, kBf16, kPrep, kOwn>), dim3((unsigned)p.stripGrid), dim3(kWaves * 64), 0,
                            stream, a);
