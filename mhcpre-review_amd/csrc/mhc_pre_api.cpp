@@ -361,7 +361,7 @@ bool slab_faster(int64_t D, int64_t T)
 }
 
 // Phase-1 knobs for tests and measurement sweeps (MHCPRE_FORCE_PATH,
-// MHCPRE_SPIN_LIMIT, MHCPRE_ROWS_B, MHCPRE_ROWS_PARTIALS, MHCPRE_SLAB) are read only when
+// MHCPRE_SPIN_LIMIT, MHCPRE_ROWS_B, MHCPRE_ROWS_PARTIALS, MHCPRE_SLAB, MHCPRE_CELL) are read only when
 // MHCPRE_TESTING=1: a stray one in a production environment changes nothing.
 const char *test_env(const char *name)
 {
@@ -1051,9 +1051,9 @@ int get_workspace(const mhcTensor *x, const mhcTensor *phi, const mhcTensor *alp
     return MHC_STATUS_SUCCESS;
 }
 
-// Co-resident workgroups of the executor's strip or fused kernel on the
+// Co-resident workgroups of one of the executor's kernels on the
 // current device: the occupancy query runs once per process, device and
-// kernel instance (n, x dtype, prepared weights, fused slice width), and its
+// kernel instance (n, x dtype, prepared weights, slice width), and its
 // result is kept in the executor too.
 int cached_coresident(std::atomic<int> &slot, int (*query)(const mhc::Plan &, int),
                       const mhc::Plan &p, int cus)
@@ -1113,7 +1113,8 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     // error an earlier call of the process may have left there (the split
     // path makes no other HIP call before its first launch).
     (void)hipGetLastError();
-    if ((p.path != mhc::Path::kSplit || p.slab.P > 0 || p.stripInstead || p.cellP > 0) && !device_shape(device, shape)) {
+    if ((p.path != mhc::Path::kSplit || p.slab.P > 0 || p.stripInstead || p.cellP > 0) &&
+        !device_shape(device, shape)) {
         return MHC_STATUS_HIP_ERROR;
     }
     const uint32_t launchId = next_launch_id();
