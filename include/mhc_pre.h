@@ -153,9 +153,12 @@ MHC_API int mhcPreGetWorkspaceSizeWithHPre(const mhcTensor *x, const mhcTensor *
  * wait expires computes what it waited for itself: such a launch is slow and
  * its outputs are right, so nothing is reported.
  *
- * A launch may be captured into a HIP graph and replayed: the exchange epoch
- * that tells the current launch's data from stale workspace contents is kept
- * in the workspace itself and advanced by every launch, replays included.
+ * A launch may be captured into a HIP graph and replayed.  What tells the
+ * current launch's exchange data from everything the workspace held before is
+ * the launch's number, which every call draws anew, and in a captured launch a
+ * count of its replays, kept in words of the library that belong to the graph
+ * (16384 captured launches of 256 workgroups; beyond that an extra node sets
+ * words of the workspace before the kernel).
  */
 MHC_API int mhcPre(void *workspace, uint64_t workspaceSize, mhcPreExecutor *executor,
            hipStream_t stream);

@@ -384,9 +384,9 @@ int device_of(const void *p)
     return attr.type == hipMemoryTypeDevice ? attr.device : -1;
 }
 
-// Launch ids (written into the status word with a timeout): process-wide,
-// strictly increasing from a start that differs between processes (time and
-// address mixed), skipping 0 and ~0.
+// Launch ids (hashed into every exchange tag, and written into the status word
+// with a timeout): process-wide, strictly increasing from a start that differs
+// between processes (time and address mixed), skipping 0 and ~0.
 uint32_t next_launch_id()
 {
     static std::atomic<uint32_t> counter{[] {
@@ -846,7 +846,7 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
             (void)hipGetLastError();
             shape = kPlanShapeDefault;
         }
-        if (shape.cus <= mhc::kMaxEpochGrid) {
+        if (shape.cus <= mhc::kMaxExchangeGrid) {
             p.slab = slab_geometry(D, T, shape);
         }
     }
@@ -1119,9 +1119,13 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     }
     const uint32_t launchId = next_launch_id();
     executor->lastLaunchId.store(launchId, std::memory_order_relaxed);
-    if (p.cellP > 0 && p.cellGrid <= mhc::kMaxEpochGrid &&
+    mhc::LaunchTag tag;
+    if (p.cellP > 0 && p.cellGrid <= mhc::kMaxExchangeGrid &&
         cached_coresident(executor->cellCoresident, mhc::cell_max_coresident, p, shape.cus) >= p.cellGrid) {
-        err = mhc::launch_cell(p, workspace, stream);
+        err = mhc::make_launch_tag(launchId, device, p.cellGrid, workspace, stream, tag);
+        if (err == hipSuccess) {
+            err = mhc::launch_cell(p, workspace, tag, stream);
+        }
         done = true;
     }
     if (!done && (p.path == mhc::Path::kStrip || p.stripInstead)) {
@@ -1139,7 +1143,7 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
         if (teamsPerXcd * geo.groups > p.stripMaxTeams && p.stripMaxTeams < p.fusedTiles) {
             teamsPerXcd = p.stripMaxTeams / geo.groups;
         }
-        if (teamsPerXcd >= 1 && shape.cus <= mhc::kMaxEpochGrid &&
+        if (teamsPerXcd >= 1 && shape.cus <= mhc::kMaxExchangeGrid &&
             cached_coresident(executor->stripCoresident, mhc::strip_max_coresident, p, shape.cus) >=
                 shape.cus) {
             mhc::Plan lp = p;
@@ -1149,7 +1153,10 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
             // Workgroups of a team beyond the slices and reducers leave at once.
             lp.stripR = mhc::strip_reducers(perXcd / teamsPerXcd - p.stripP);
             lp.stripGrid = shape.cus;
-            err = mhc::launch_strip(lp, workspace, launchId, stream);
+            err = mhc::make_launch_tag(launchId, device, lp.stripGrid, workspace, stream, tag);
+            if (err == hipSuccess) {
+                err = mhc::launch_strip(lp, workspace, tag, launchId, stream);
+            }
             done = true;
         }
     }
@@ -1169,15 +1176,21 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
         if (coresident >= p.fusedP) {
             mhc::Plan lp = p;
             lp.statusWord = executor->statusWord.load(std::memory_order_relaxed);
-            lp.fusedTeams = std::min(coresident, mhc::kMaxEpochGrid) / p.fusedP;
+            lp.fusedTeams = std::min(coresident, mhc::kMaxExchangeGrid) / p.fusedP;
             lp.fusedGrid = lp.fusedTeams * p.fusedP;
-            err = mhc::launch_fused(lp, workspace, launchId, stream);
+            err = mhc::make_launch_tag(launchId, device, lp.fusedGrid, workspace, stream, tag);
+            if (err == hipSuccess) {
+                err = mhc::launch_fused(lp, workspace, tag, launchId, stream);
+            }
             done = true;
         }
     }
     if (!done && p.slab.P > 0 && p.slab.grid == shape.cus && p.slab.xcds == shape.xcds &&
         cached_coresident(executor->slabCoresident, mhc::slab_max_coresident, p, shape.cus) >= shape.cus) {
-        err = mhc::launch_slab(p, workspace, stream);
+        err = mhc::make_launch_tag(launchId, device, p.slab.grid, workspace, stream, tag);
+        if (err == hipSuccess) {
+            err = mhc::launch_slab(p, workspace, tag, stream);
+        }
         done = true;
     }
     if (!done && p.path == mhc::Path::kRows) {
@@ -1193,10 +1206,10 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     return err == hipSuccess ? MHC_STATUS_SUCCESS : MHC_STATUS_HIP_ERROR;
 }
 
-// The occupancy queries of a new executor and the address of the device's
-// built-in workspace (mhcPreNoAlloc), when the current device is the one
+// The occupancy queries of a new executor and the addresses of the device's
+// built-in workspace (mhcPreNoAlloc) and replay words, when the current device is the one
 // that holds its tensors (otherwise its first launch makes them): so that a
-// later launch, one under stream capture included, makes neither call.
+// later launch, one under stream capture included, makes none of these calls.
 void prime_coresident(mhcPreExecutor *ex)
 {
     const mhc::Plan &p = ex->plan;
@@ -1211,6 +1224,12 @@ void prime_coresident(mhcPreExecutor *ex)
     }
     void *scratch = nullptr;
     if (mhc::scratch_address(device, &scratch) != hipSuccess) {
+        (void)hipGetLastError();
+    }
+    const bool exchanges = p.cellP > 0 || p.stripInstead || p.slab.P > 0 || p.path == mhc::Path::kStrip ||
+                           p.path == mhc::Path::kFused;
+    uint32_t *words = nullptr;
+    if (exchanges && mhc::replay_words_address(device, &words) != hipSuccess) {
         (void)hipGetLastError();
     }
     if (p.cellP > 0) {

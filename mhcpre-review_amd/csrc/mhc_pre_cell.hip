@@ -30,9 +30,9 @@
 // bytes alone take under 1 us.
 //
 // Every record word is 8 bytes, the fp32 bits and a tag (a hash of the word's
-// position XOR the launch's epoch, which the workspace header keeps), read and
-// written as one access at device scope; a word is current exactly when its
-// tag matches, so the workspace needs no clearing.  The grid is at most what
+// position XOR the launch's epoch, see launch_epoch), read and written as one
+// access at device scope; a word is current exactly when its tag matches, so
+// the workspace needs no clearing.  The grid is at most what
 // the device holds at once.  Waits are bounded: a workgroup whose wait expires
 // (another kernel holds the CUs that the rest needs) computes every slice's
 // sums itself, in the order of the exchange, so such a launch is slow and its
@@ -79,7 +79,7 @@ struct CellArgs {
     float *hRes;
     float *hPre;
     uint64_t *recs;  // [column tile][row tile][P] records
-    char *hdr;       // workspace header
+    LaunchTag tag;
     int T;
     int D;
     int K;
@@ -110,13 +110,13 @@ __global__ __launch_bounds__((Cell<N, NS>::kThreads), (Cell<N, NS>::kWavesPerSim
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t prevEpoch = tid == 0 ? epoch_load(a.hdr, kWsEpochOff) : 0u;
     const int P = a.P;
     // Column tile 0 first: its workgroups' wait is the longest way.
     const int p = blockIdx.x;
     const int tile = blockIdx.y;
     const int ct = blockIdx.z;
     const int group = ct * (int)gridDim.y + tile;
+    const uint32_t replays = tid == 0 ? replay_load(a.tag.words, group * P + p) : 0u;
     const bool half = (M & 15) != 0 && ct == Q;  // 8 columns; lanes 8-15 of a row of 16 repeat them
     const int s = w % N;       // the wave's stream
     const int strip = w / N;   // and strip
@@ -273,8 +273,7 @@ __global__ __launch_bounds__((Cell<N, NS>::kThreads), (Cell<N, NS>::kWavesPerSim
         }
     }
     if (tid == 0) {
-        epochSh = epoch_next(prevEpoch);
-        epoch_mark(a.hdr, kWsSeenOff, epochSh, group * P + p);
+        epochSh = launch_epoch<CellArgs>(group * P + p, replays);
     }
     lds_barrier();
     const uint32_t epoch = __builtin_amdgcn_readfirstlane(epochSh);
@@ -448,11 +447,6 @@ __global__ __launch_bounds__((Cell<N, NS>::kThreads), (Cell<N, NS>::kWavesPerSim
         store16<kCpolNt>(out, make_rsrc(a.hIn + (int64_t)tile * 16 * Di, rows * Di * 2),
                          col < Di ? (row * Di + col) * 2 : kPast);
     }
-    // Workgroup 0 advances the workspace's epoch once every workgroup has
-    // taken this one; its last wave (which has no part in hIn) waits for that.
-    if (group == 0 && p == 0 && w == W - 1) {
-        (void)epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, P * (int)(gridDim.y * gridDim.z), kPublishPolls);
-    }
 }
 
 template <int N, int NS, bool kBf16, bool kPrep>
@@ -467,7 +461,7 @@ struct Instance {
         }
         return perCU * numCUs;
     }
-    static hipError_t launch(const Plan &p, void *workspace, hipStream_t stream)
+    static hipError_t launch(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
     {
         char *ws = static_cast<char *>(workspace);
         CellArgs a;
@@ -482,7 +476,7 @@ struct Instance {
         a.hRes = p.hRes;
         a.hPre = p.hasHPre ? p.hPre : nullptr;
         a.recs = reinterpret_cast<uint64_t *>(ws + p.wsCellRecs);
-        a.hdr = ws;
+        a.tag = tag;
         a.T = (int)p.T;
         a.D = (int)p.D;
         a.K = (int)p.K;
@@ -531,9 +525,9 @@ int cell_max_coresident(const Plan &p, int numCUs)
     return with_instance(p, [&](auto i) { return decltype(i)::coresident(numCUs); });
 }
 
-hipError_t launch_cell(const Plan &p, void *workspace, hipStream_t stream)
+hipError_t launch_cell(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
 {
-    return with_instance(p, [&](auto i) { return decltype(i)::launch(p, workspace, stream); });
+    return with_instance(p, [&](auto i) { return decltype(i)::launch(p, workspace, tag, stream); });
 }
 
 }  // namespace mhc

@@ -8,6 +8,7 @@
 #include <utility>
 
 #include "mhc_pre.h"
+#include "mhc_pre_internal.h"
 
 namespace mhc {
 namespace dev {
@@ -271,69 +272,39 @@ __device__ __forceinline__ void split_f16_to_bf16(const float (&f)[8], u32x4_t &
     }
 }
 
-// Exchange epoch of a strip or fused launch, kept in the workspace header.
-// One thread of every workgroup reads the epoch the previous launch on the
-// workspace stored (epoch_load); the launch uses epoch_next of it, so
-// consecutive launches on a workspace, graph replays included, never share an
-// epoch.  Each workgroup records the epoch it uses in its own slot
-// (epoch_mark); one wave of workgroup 0 stores the new epoch at its end, once
-// every workgroup's slot holds it (epoch_publish), so no workgroup can read
-// the advanced value.  No workgroup contends for a word, and a workspace left
-// with any contents by other use needs no reset.
-__device__ __forceinline__ uint32_t epoch_next(uint32_t prev)
+// The kernel's arguments, read again from the kernarg segment.  (Taken from the
+// parameter, all of them stay in scalar registers from the start of the kernel
+// to their last use, and large kernels spill.)
+template <typename Args>
+__device__ __forceinline__ const __attribute__((address_space(4))) Args *late_args()
 {
-    const uint32_t e = prev + 1u;
-    return (e == 0u || e == 0xFFFFFFFFu) ? 1u : e;  // 0 and ~0 never tag a word
+    auto *p = (const __attribute__((address_space(4))) Args *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t header_rsrc(void *ws, size_t off, int bytes)
+// The epoch of a launch, mixed into every exchange word's tag: the launch tag's
+// seed, and in a captured launch the replays this workgroup has counted in its
+// own word of the tag's.  One thread of every workgroup that the launch has
+// (spare ones too, the words stay equal) calls replay_load early and
+// launch_epoch once, later.
+__device__ __forceinline__ uint32_t replay_load(uint32_t *words, int g)
 {
-    return __builtin_amdgcn_make_buffer_rsrc(static_cast<char *>(ws) + off, (short)0, bytes, 0x00020000);
+    return words == nullptr
+               ? 0u
+               : (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(make_rsrc(words + g, 4), 0, 0, kCpolDev);
 }
 
-__device__ __forceinline__ uint32_t epoch_load(void *ws, size_t epochOff)
+template <typename Args>
+__device__ __forceinline__ uint32_t launch_epoch(int g, uint32_t loaded)
 {
-    return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(header_rsrc(ws, epochOff, 4), 0, 0, 16 /* sc1 */);
-}
-
-__device__ __forceinline__ void epoch_mark(void *ws, size_t seenOff, uint32_t epoch, int g)
-{
-    __builtin_amdgcn_raw_buffer_store_b32(epoch, header_rsrc(ws, seenOff, 4 * (g + 1)), 4 * g, 0,
-                                          16 /* sc1 */);
-}
-
-// epoch_publish's limit in kernels whose other waits are shorter (about a
-// second): their late workgroups must not read the advanced epoch.
-constexpr uint32_t kPublishPolls = 1u << 20;
-
-// One whole wave: waits (bounded by spinLimit polls) until the slots of all
-// `grid` workgroups hold `epoch`, then stores it as the header's epoch.
-// Returns false if the wait expired (the epoch is stored anyway, so that the
-// next launch cannot reuse it).
-__device__ __forceinline__ bool epoch_publish(void *ws, size_t epochOff, size_t seenOff, uint32_t epoch,
-                                              int grid, uint32_t spinLimit)
-{
-    const int lane = (int)(threadIdx.x & 63);
-    const __amdgpu_buffer_rsrc_t seen = header_rsrc(ws, seenOff, 4 * grid);
-    bool done = false;
-    for (uint32_t spins = 0;; ++spins) {
-        bool ok = true;
-        for (int i = lane; i < grid; i += 64) {
-            ok = ok && (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(seen, 4 * i, 0, 16) == epoch;
-        }
-        if (__all(ok)) {
-            done = true;
-            break;
-        }
-        if (spins >= spinLimit) {
-            break;
-        }
-        __builtin_amdgcn_s_sleep(2);
+    const auto *a = late_args<Args>();
+    uint32_t *words = a->tag.words;
+    if (words == nullptr) {
+        return a->tag.seed;
     }
-    if (lane == 0) {
-        __builtin_amdgcn_raw_buffer_store_b32(epoch, header_rsrc(ws, epochOff, 4), 0, 0, 16);
-    }
-    return done;
+    __builtin_amdgcn_raw_buffer_store_b32(loaded + 1u, make_rsrc(words + g, 4), 0, 0, kCpolDev);
+    return a->tag.seed ^ mix32(loaded + 1u);
 }
 
 // Quiet NaN written into the outputs of rows whose exchange wait expired.

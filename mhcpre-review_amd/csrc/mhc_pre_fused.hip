@@ -39,9 +39,8 @@
 // no reset of the workspace between launches.  A reader accepts a block only
 // when every word it read carries the expected tag; a block left over from an
 // earlier launch (another epoch) or filled with any constant never does.  The
-// epoch is kept in the workspace header (epoch_load / mark / publish), so the
-// replays of a captured HIP graph get fresh epochs too.  Every wait is bounded
-// by a spin limit; running out records kDeviceTimeout with the host launch id
+// epoch is launch_epoch's, which no other launch or replay has.  Every wait is
+// bounded by a spin limit; running out records kDeviceTimeout with the host launch id
 // in the status word instead of hanging, and the values that wait was for are
 // taken as NaN, so the affected outputs are NaN.  The grid is
 // sized to the device's co-residency limit, so every workgroup is resident
@@ -78,7 +77,7 @@ struct FusedArgs {
     uint64_t *recs;      // [RT][P] records of Rec<N>::WORDS tagged words
     uint64_t *bcast;     // [RT] blocks of Rec<N>::BWORDS tagged words
     uint64_t *status;    // (launchId << 32) | kDeviceTimeout after a timeout
-    char *hdr;           // workspace header (status word, exchange epoch)
+    LaunchTag tag;
     uint32_t *statusWord;  // the caller's sticky status word, or null
     int64_t T;
     int64_t D;
@@ -230,14 +229,13 @@ __global__ __launch_bounds__(kFusedWaves * 64) void fused_kernel(FusedArgs a)
     static_assert(N == 4, "the fused path maps the n = 4 hPre columns to the 4 lane groups");
 
     const int tid = threadIdx.x;
-    // Thread 0 reads the epoch the previous launch on this workspace left.
-    const uint32_t prevEpoch = tid == 0 ? epoch_load(a.hdr, kWsEpochOff) : 0u;
     const int P = a.P;
     const int numTeams = a.numTeams;
     const int g = blockIdx.x;
+    const uint32_t replays = tid == 0 ? replay_load(a.tag.words, g) : 0u;
     if (g >= P * numTeams) {
         if (tid == 0) {
-            epoch_mark(a.hdr, kWsSeenOff, epoch_next(prevEpoch), g);
+            (void)launch_epoch<FusedArgs>(g, replays);
         }
         return;  // spare workgroup: the whole workgroup leaves together
     }
@@ -266,7 +264,7 @@ __global__ __launch_bounds__(kFusedWaves * 64) void fused_kernel(FusedArgs a)
     };
     if ((int64_t)team * W >= a.RT) {
         if (tid == 0) {
-            epoch_mark(a.hdr, kWsSeenOff, epoch_next(prevEpoch), g);
+            (void)launch_epoch<FusedArgs>(g, replays);
         }
         return;  // no row tile for any wave of this workgroup
     }
@@ -366,8 +364,7 @@ __global__ __launch_bounds__(kFusedWaves * 64) void fused_kernel(FusedArgs a)
     }
 
     if (tid == 0) {
-        epochSh = epoch_next(prevEpoch);
-        epoch_mark(a.hdr, kWsSeenOff, epochSh, g);
+        epochSh = launch_epoch<FusedArgs>(g, replays);
     }
     __syncthreads();
 
@@ -696,13 +693,6 @@ __global__ __launch_bounds__(kFusedWaves * 64) void fused_kernel(FusedArgs a)
     if (prevTile >= 0) {
         post_res(prevTile, prevInvRms, P, lane);
     }
-    // Workgroup 0 (team 0, which always has a tile) advances the workspace's
-    // epoch once every workgroup has taken this one.
-    if (g == 0 && wave == 0) {
-        if (!epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, a.spinLimit)) {
-            record_timeout(a, lane);
-        }
-    }
 }
 
 template <int N, int KP, bool kBf16, bool kPrep>
@@ -742,7 +732,8 @@ int fused_coresident_t(int numCUs)
 }
 
 template <int N, int KP, bool kBf16, bool kPrep>
-hipError_t launch_fused_t(const Plan &p, void *workspace, uint32_t launchId, hipStream_t stream)
+hipError_t launch_fused_t(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId,
+                          hipStream_t stream)
 {
     hipError_t err = fused_prepare_attr<N, KP, kBf16, kPrep>();
     if (err != hipSuccess) {
@@ -762,7 +753,7 @@ hipError_t launch_fused_t(const Plan &p, void *workspace, uint32_t launchId, hip
     a.hPre = p.hasHPre ? p.hPre : nullptr;
     a.status = reinterpret_cast<uint64_t *>(ws);
     a.statusWord = p.statusWord;
-    a.hdr = ws;
+    a.tag = tag;
     a.bcast = reinterpret_cast<uint64_t *>(ws + p.wsFinal);
     a.recs = reinterpret_cast<uint64_t *>(ws + p.wsFusedPartial);
     a.T = p.T;
@@ -811,12 +802,13 @@ hipError_t launch_fused_t(const Plan &p, void *workspace, uint32_t launchId, hip
         MHC_FUSED_DISPATCH_P(FN, false, __VA_ARGS__)                           \
     }
 
-hipError_t launch_fused(const Plan &p, void *workspace, uint32_t launchId, hipStream_t stream)
+hipError_t launch_fused(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId,
+                          hipStream_t stream)
 {
     if (p.n != 4) {
         return hipErrorNotSupported;
     }
-    MHC_FUSED_DISPATCH(launch_fused_t, p, workspace, launchId, stream)
+    MHC_FUSED_DISPATCH(launch_fused_t, p, workspace, tag, launchId, stream)
     return hipErrorNotSupported;
 }
 

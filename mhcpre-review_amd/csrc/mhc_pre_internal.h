@@ -22,18 +22,41 @@ enum class Path : int {
 constexpr uint32_t kDeviceOk = 0u;
 constexpr uint32_t kDeviceTimeout = 0x7107u;
 
-// Bytes reserved at the head of the workspace: the status word at 0, and the
-// exchange epoch of the strip and fused kernels.  The epoch lives in device
-// memory, not in the kernel arguments, so that a launch captured in a HIP
-// graph still gets a fresh epoch on every replay: every workgroup reads the
-// word at kWsEpochOff, uses one more than it and records the epoch it uses in
-// its own slot of the array at kWsSeenOff; workgroup 0, at its end, stores
-// the new epoch once every slot of the grid holds it (no workgroup reads the
-// word after that).
-constexpr size_t kWsEpochOff = 64;            // uint32: epoch of the latest strip / fused launch
-constexpr size_t kWsSeenOff = 256;            // uint32 [kMaxEpochGrid]: epoch each workgroup uses
-constexpr int kMaxEpochGrid = 2048;           // largest strip / fused grid
-constexpr size_t kWsHeaderBytes = kWsSeenOff + 4 * kMaxEpochGrid;
+// Bytes reserved at the head of the workspace: the status word at 0, and words
+// that only launches captured when the library's own were used up need
+// (mhc_pre_replay.hip).
+constexpr size_t kWsReplayOff = 256;  // uint32 [kMaxExchangeGrid]
+constexpr int kMaxExchangeGrid = 2048;  // largest grid of a kernel whose workgroups exchange words
+constexpr size_t kWsHeaderBytes = kWsReplayOff + 4 * kMaxExchangeGrid;
+
+// What the kernels whose workgroups exchange words (cell, slab, strip, fused)
+// mix into every tag, so that no word of another launch is taken for one of
+// this launch's, whatever the workspace held before: a hash of the launch's
+// number, which no two launches of a process share.  The replays of a captured
+// launch share it; `words` (null for an eager launch) then holds one word per
+// workgroup, equal in all of them, to which each replay adds one.
+struct LaunchTag {
+    uint32_t seed = 0;
+    uint32_t *words = nullptr;
+};
+
+// The finalizer of MurmurHash3 (a bijection): distinct numbers, distinct
+// seeds, and the seeds of neighbouring launches differ in half their bits.
+__host__ __device__ inline uint32_t mix32(uint32_t v)
+{
+    v ^= v >> 16;
+    v *= 0x85EBCA6Bu;
+    v ^= v >> 13;
+    v *= 0xC2B2AE35u;
+    return v ^ (v >> 16);
+}
+
+// The tag of launch `launchId` with `grid` workgroups, on the current device
+// `device` (mhc_pre_replay.hip).
+hipError_t make_launch_tag(uint32_t launchId, int device, int grid, void *workspace, hipStream_t stream,
+                           LaunchTag &tag);
+// The current device's array of replay words (looked up once per device).
+hipError_t replay_words_address(int device, uint32_t **ptr);
 
 // Work distribution of the slab kernel (mhc_pre_slab.hip).
 struct SlabGeometry {
@@ -182,17 +205,17 @@ hipError_t launch_split(const Plan &plan, void *workspace, hipStream_t stream);
 // launchId: host-side id of the launch, written with kDeviceTimeout into the
 // status word when a bounded wait expires (the exchange epoch itself comes
 // from the workspace header).
-hipError_t launch_fused(const Plan &plan, void *workspace, uint32_t launchId, hipStream_t stream);
+hipError_t launch_fused(const Plan &plan, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream);
 
-hipError_t launch_strip(const Plan &plan, void *workspace, uint32_t launchId, hipStream_t stream);
+hipError_t launch_strip(const Plan &plan, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream);
 
 // Cell kernel (mhc_pre_cell.hip).
-hipError_t launch_cell(const Plan &plan, void *workspace, hipStream_t stream);
+hipError_t launch_cell(const Plan &plan, void *workspace, const LaunchTag &tag, hipStream_t stream);
 int cell_max_coresident(const Plan &plan, int numCUs);
 size_t cell_record_bytes();
 
 // Slab kernel (mhc_pre_slab.hip): one launch, x read once.
-hipError_t launch_slab(const Plan &plan, void *workspace, hipStream_t stream);
+hipError_t launch_slab(const Plan &plan, void *workspace, const LaunchTag &tag, hipStream_t stream);
 int slab_max_coresident(const Plan &plan, int numCUs);
 int slab_columns();                          // x columns per slice
 int slab_max_slices();                       // largest P

@@ -9,9 +9,8 @@
 // device address) but the address hipGetSymbolAddress returns for the current
 // device, looked up once per device.  Every launch on a device shares that
 // device's copy and finds the previous launch's contents there; the kernels
-// need nothing in it to start at zero (the exchange tags carry an epoch kept
-// in the array's header, the split-K partials are written before they are
-// read).  Launches that overlap on one device race on the array.
+// need nothing in it to start at zero (the exchange tags differ in every
+// launch, the split-K partials are written before they are read).  Launches that overlap on one device race on the array.
 
 #include "mhc_pre_internal.h"
 

@@ -41,11 +41,10 @@
 // hPre columns) and every flag is an 8-byte word: the fp32 bits and a tag (a
 // hash of the word's position XOR the launch's epoch), read and written as one
 // access; a word is current exactly when its tag matches, so nothing is
-// counted, reset or cleared.  The epoch is kept in the workspace header
-// (epoch_load and epoch_publish), so graph replays get fresh ones.  The hPost
-// and hRes columns, five sixths of a record, are plain values: a wave stores
-// its flag for step m an own step later, when a counter wait has shown that
-// its stores of m are done, and readers look at the flag first.
+// counted, reset or cleared.  The epoch is launch_epoch's: no other launch has
+// it.  The hPost and hRes columns, five sixths of a record, are plain values:
+// a wave stores its flag for step m an own step later, when a counter wait has
+// shown that its stores of m are done, and readers look at the flag first.
 //
 // Reducers.  The waves of a team's reducer workgroups work alone, one tile at
 // a time, without barriers: a tile's reduction is a chain of memory round
@@ -137,7 +136,7 @@ struct SlabArgs {
     uint64_t *flags;  // [team][S][P][2] words: strip 0 and 1 of the slice have stored their plain columns
     uint64_t *bcast;  // [team][S] broadcast blocks
     uint64_t *done;   // [team][kMaxRest] words: the latest step a wave has finished reading
-    char *hdr;        // workspace header
+    LaunchTag tag;
     int64_t T;
     int64_t D;
     int64_t K;
@@ -154,17 +153,9 @@ struct SlabArgs {
     uint32_t spinLimit;
 };
 
-// The kernel's arguments, read again from the kernarg segment: each phase of
-// the kernel loads the ones that it uses.  (Taken from the parameter, all of
-// them stay in scalar registers from the start of the kernel to its end, and
-// the slice loop spills.)
+// (Each phase of the kernel loads the arguments that it uses.)
 typedef const __attribute__((address_space(4))) SlabArgs *ArgsPtr;
-__device__ __forceinline__ ArgsPtr phase_args()
-{
-    ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return p;
-}
+__device__ __forceinline__ ArgsPtr phase_args() { return late_args<SlabArgs>(); }
 
 __device__ __forceinline__ WeightsRef weights_of(ArgsPtr p) { return {p->phi, p->gamma, p->bprep, (int)p->K}; }
 
@@ -499,7 +490,7 @@ __global__ __launch_bounds__(kThreads) void slab_kernel(SlabArgs a)
 
     const int tid = threadIdx.x;
     const int g = blockIdx.x;
-    const uint32_t prevEpoch = tid == 0 ? epoch_load(a.hdr, kWsEpochOff) : 0u;
+    const uint32_t replays = tid == 0 ? replay_load(a.tag.words, g) : 0u;
     const int xcd = g % a.nGroups;
     const int jg = g / a.nGroups;
     const int teamSize = a.P + a.R;
@@ -508,15 +499,14 @@ __global__ __launch_bounds__(kThreads) void slab_kernel(SlabArgs a)
     const int numTeams = a.nGroups * a.perGroup;
     const int ntiles = tj < a.perGroup && team < a.RT ? (a.RT - team + numTeams - 1) / numTeams : 0;
     if (tid == 0) {
-        epochSh = epoch_next(prevEpoch);
-        epoch_mark(a.hdr, kWsSeenOff, epochSh, g);
+        epochSh = launch_epoch<SlabArgs>(g, replays);
     }
     if (tid < kGroups) {
         arrived[tid] = 0;
         taken[tid] = 0;
     }
     if (ntiles == 0) {
-        return;  // a spare workgroup, or a team without tiles (never workgroup 0)
+        return;  // a spare workgroup, or a team without tiles
     }
     const int role = jg % teamSize;
     const int lane = tid & 63;
@@ -1003,12 +993,6 @@ __global__ __launch_bounds__(kThreads) void slab_kernel(SlabArgs a)
             }
         }
     }
-    // Workgroup 0 (a slice of team 0) advances the workspace's epoch once
-    // every workgroup has taken this one.
-    if (g == 0 && w == 0) {
-        const ArgsPtr ea = phase_args();
-        (void)epoch_publish(ea->hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, kPublishPolls);
-    }
 }
 
 template <int N, bool kBf16, bool kPrep>
@@ -1024,7 +1008,7 @@ int slab_coresident_t(int numCUs)
 }
 
 template <int N, bool kBf16, bool kPrep>
-hipError_t launch_slab_t(const Plan &p, void *workspace, hipStream_t stream)
+hipError_t launch_slab_t(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
 {
     char *ws = static_cast<char *>(workspace);
     SlabArgs a;
@@ -1042,7 +1026,7 @@ hipError_t launch_slab_t(const Plan &p, void *workspace, hipStream_t stream)
     a.bcast = reinterpret_cast<uint64_t *>(ws + p.wsSlabBcast);
     a.flags = reinterpret_cast<uint64_t *>(ws + p.wsSlabFlags);
     a.done = reinterpret_cast<uint64_t *>(ws + p.wsSlabDone);
-    a.hdr = ws;
+    a.tag = tag;
     a.T = p.T;
     a.D = p.D;
     a.K = p.K;
@@ -1087,17 +1071,17 @@ int slab_max_coresident(const Plan &p, int numCUs)
     return p.isBf16 ? slab_coresident_t<6, true, false>(numCUs) : slab_coresident_t<6, false, false>(numCUs);
 }
 
-hipError_t launch_slab(const Plan &p, void *workspace, hipStream_t stream)
+hipError_t launch_slab(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
 {
     if (p.n != 6) {
         return hipErrorNotSupported;
     }
     if (p.bprep != nullptr) {
-        return p.isBf16 ? launch_slab_t<6, true, true>(p, workspace, stream)
-                        : launch_slab_t<6, false, true>(p, workspace, stream);
+        return p.isBf16 ? launch_slab_t<6, true, true>(p, workspace, tag, stream)
+                        : launch_slab_t<6, false, true>(p, workspace, tag, stream);
     }
-    return p.isBf16 ? launch_slab_t<6, true, false>(p, workspace, stream)
-                    : launch_slab_t<6, false, false>(p, workspace, stream);
+    return p.isBf16 ? launch_slab_t<6, true, false>(p, workspace, tag, stream)
+                    : launch_slab_t<6, false, false>(p, workspace, tag, stream);
 }
 
 }  // namespace mhc

@@ -47,10 +47,9 @@
 // atomic accesses at device scope (sc1).  The tag is a hash of the word's
 // position XOR a per-launch epoch, so a word holds the current value exactly
 // when its tag matches: no arrival counter, no release wait, no reset of the
-// workspace between launches.  The epoch is kept in the workspace header
-// (epoch_load / epoch_mark / epoch_publish), so replays of a captured HIP graph get fresh
-// epochs too.  Every wait is bounded by a spin limit; running out records
-// kDeviceTimeout with the host launch id in the status word instead of
+// workspace between launches.  The epoch is launch_epoch's, which no other
+// launch or replay has.  Every wait is bounded by a spin limit; running out
+// records kDeviceTimeout with the host launch id in the status word instead of
 // hanging, and the rows the wave or workgroup could not finish get NaN
 // outputs.  The grid is one workgroup per CU, all co-resident when nothing
 // else occupies the device.
@@ -107,7 +106,7 @@ struct StripArgs {
     uint64_t *recs;    // [team][ringSlots][P] records of Rec<N>::WORDS tagged words
     uint64_t *bcast;   // [team][ringSlots] blocks of Rec<N>::BWORDS tagged words
     char *hdr;         // workspace header: the status word ((launchId << 32) |
-                       // kDeviceTimeout after a timeout) at 0, the exchange epoch
+                       // kDeviceTimeout after a timeout) at 0
     uint32_t *statusWord;  // the caller's sticky status word, or null
     int64_t T;
     int64_t D;
@@ -123,6 +122,7 @@ struct StripArgs {
     float invFlatDim;
     uint32_t launchId;
     uint32_t spinLimit;
+    LaunchTag tag;
 };
 
 // Column slots of the [hi | lo] B operand, NT = 2M/16 tiles of 16 lanes:
@@ -197,11 +197,13 @@ __device__ __forceinline__ void st_status(uint64_t *status, uint32_t launchId)
                                           make_rsrc(status, 8), 0, 0, kCpolDev);
 }
 
-__device__ __forceinline__ void record_timeout(const StripArgs &a, int lane)
+typedef const __attribute__((address_space(4))) StripArgs *ArgsPtr;
+
+__device__ __forceinline__ void record_timeout(ArgsPtr a, int lane)
 {
     if (lane == 0) {
-        st_status(reinterpret_cast<uint64_t *>(a.hdr), a.launchId);
-        st_status_word(a.statusWord);
+        st_status(reinterpret_cast<uint64_t *>(a->hdr), a->launchId);
+        st_status_word(a->statusWord);
     }
 }
 
@@ -287,8 +289,8 @@ struct ColPoll {
 };
 
 template <int N, int MaxS, bool kBf16, bool kOwn>
-__device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int ntiles, int r, int R,
-                                           bool local, float *lds, uint32_t prevEpoch,
+__device__ __forceinline__ void reducer_wg(int team, int ntiles, int r, int R,
+                                           bool local, float *lds, uint32_t replays,
                                            uint32_t *epochSh)
 {
     using RC = Rec<N>;
@@ -307,28 +309,29 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
     static_assert(8 * (N + 1) <= 64, "phase 1 is finished by one wave");
     uint32_t voteParity = 0;
     const int tid = threadIdx.x;
-    const int P = a.P;
-    // The launch's exchange epoch: read by thread 0 from the workspace header
-    // (prevEpoch), handed to every wave through LDS.
+    // (The arguments are read again for each tile: see late_args.)
+    const ArgsPtr first = late_args<StripArgs>();
+    const int P = first->P;
+    // The launch's exchange epoch, handed from thread 0 to every wave.
     if (tid == 0) {
-        *epochSh = epoch_next(prevEpoch);
-        epoch_mark(a.hdr, kWsSeenOff, *epochSh, blockIdx.x);
+        *epochSh = launch_epoch<StripArgs>(blockIdx.x, replays);
     }
     lds_barrier();
     const uint32_t epoch = __builtin_amdgcn_readfirstlane(*epochSh);
-    const float alphaPre = a.alpha[0];
-    const float alphaPost = a.alpha[1];
-    const float alphaRes = a.alpha[2];
+    const float alphaPre = first->alpha[0];
+    const float alphaPost = first->alpha[1];
+    const float alphaRes = first->alpha[2];
     Poll1 p1(tid);
     Poll2 p2(tid);
     // The bias of this thread's column in each phase, loaded once.
-    const float bias1 = a.bias[p1.c < N ? p1.c : 0];
-    const float bias2 = a.bias[p2.c - 1];
+    const float bias1 = first->bias[p1.c < N ? p1.c : 0];
+    const float bias2 = first->bias[p2.c - 1];
     bool timedOut = false;
     // kOwn: the sums of mix columns j0 .. j1 - 1 (and, with j0 = 0, the sum of
     // squares) of a tile whose records did not come, into group 0 of `sums`
     // (the others zero), a wave per row.
     const auto own_phase = [&](int rt, int j0, int j1) {
+        const ArgsPtr a = late_args<StripArgs>();
         const int items = j0 == 0 ? Poll1::ITEMS : Poll2::ITEMS;
         const int groups = j0 == 0 ? Poll1::SG : Poll2::SG;
         __syncthreads();
@@ -341,8 +344,8 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
 #pragma unroll 1
             for (int j = j0; j < j1; j += 8) {
                 float own[9];
-                own_sums<N, kBf16>(WeightsRef{a.phi, a.gamma, a.bprep, (int)a.K}, a.x, a.T, (int64_t)rt * 16 + row, j,
-                                   own);
+                own_sums<N, kBf16>(WeightsRef{a->phi, a->gamma, a->bprep, (int)a->K}, a->x, a->T,
+                                   (int64_t)rt * 16 + row, j, own);
                 // Item (column j - j0) * 8 + row / 2 of the phase, component
                 // row % 2; the sum of squares is phase 1's last column.
                 const int at = 2 * (row >> 1) + (row & 1);
@@ -362,9 +365,10 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
         __syncthreads();
     };
     for (int k = r; k < ntiles; k += R) {
-        const int rt = team + a.numTeams * k;
+        const ArgsPtr a = late_args<StripArgs>();
+        const int rt = team + a->numTeams * k;
         const uint32_t slot = (uint32_t)(team * kRingSlots + k % kRingSlots);
-        const __amdgpu_buffer_rsrc_t tr = make_rsrc(a.recs + (uint64_t)slot * P * RC::WORDS, P * RC::WORDS * 8);
+        const __amdgpu_buffer_rsrc_t tr = make_rsrc(a->recs + (uint64_t)slot * P * RC::WORDS, P * RC::WORDS * 8);
         const uint32_t tileBase = (uint32_t)rt * (uint32_t)P * (uint32_t)RC::WORDS;
 
         // Phase 1: hPre columns and sum of squares.  Once a wait of this
@@ -382,7 +386,7 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
             if (timedOut) {
                 break;  // an earlier wait expired: no more waiting in this launch
             }
-            if (spins >= a.spinLimit) {
+            if (spins >= a->spinLimit) {
                 if constexpr (!kOwn) {
                     record_timeout(a, tid);
                 }
@@ -424,8 +428,8 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
             }
             float ir2[2] = {0.f, 0.f};
             if (tid < Poll1::ITEMS && p1.c == N) {  // sum of squares: invRms of rows r0, r0 + 1
-                ir2[0] = ref_inv_rms(tot.x, a.invFlatDim, a.normEps);
-                ir2[1] = ref_inv_rms(tot.y, a.invFlatDim, a.normEps);
+                ir2[0] = ref_inv_rms(tot.x, a->invFlatDim, a->normEps);
+                ir2[1] = ref_inv_rms(tot.y, a->invFlatDim, a->normEps);
                 irs[p1.r0] = ir2[0];
                 irs[p1.r0 + 1] = ir2[1];
             }
@@ -440,16 +444,16 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
             for (int e = 0; e < 2; ++e) {
                 const float ir = ir2[e];
                 const float mix = e == 0 ? tot.x : tot.y;
-                const float v = ref_sigmoid(mix * (ir * alphaPre), bias1, a.hcEps);
+                const float v = ref_sigmoid(mix * (ir * alphaPre), bias1, a->hcEps);
                 const int idx = c * 16 + p1.r0 + e;
                 wv[2 * e] = __float_as_uint(v);
                 wv[2 * e + 1] = bcast_tag((uint32_t)rt * (uint32_t)RC::BWORDS + (uint32_t)idx, epoch);
                 const int row = rt * 16 + p1.r0 + e;
-                if (a.hPre != nullptr && row < a.T) {
-                    a.hPre[(int64_t)row * N + c] = v;
+                if (a->hPre != nullptr && row < a->T) {
+                    a->hPre[(int64_t)row * N + c] = v;
                 }
             }
-            const __amdgpu_buffer_rsrc_t br = make_rsrc(a.bcast + (uint64_t)slot * RC::BWORDS, RC::BWORDS * 8);
+            const __amdgpu_buffer_rsrc_t br = make_rsrc(a->bcast + (uint64_t)slot * RC::BWORDS, RC::BWORDS * 8);
             if (local) {
                 store16<0>(wv, br, (c * 16 + p1.r0) * 8);
             } else {
@@ -470,7 +474,7 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
             if (timedOut) {
                 break;
             }
-            if (spins >= a.spinLimit) {
+            if (spins >= a->spinLimit) {
                 if constexpr (!kOwn) {
                     record_timeout(a, tid);
                 }
@@ -511,13 +515,13 @@ __device__ __forceinline__ void reducer_wg(const StripArgs &a, int team, int nti
                 const int row = rt * 16 + p2.r0 + e;
                 const float v = e == 0 ? tot.x : tot.y;
                 const float ir = irs[p2.r0 + e];
-                if (row < a.T) {
+                if (row < a->T) {
                     if (jj < 2 * N) {
                         const float sgm = ref_sigmoid(v * (ir * alphaPost), bias2, 0.0f);
-                        a.hPost[(int64_t)row * N + (jj - N)] = sgm * 2.0f;
+                        a->hPost[(int64_t)row * N + (jj - N)] = sgm * 2.0f;
                     } else {
                         const float rr = v * (ir * alphaRes);
-                        a.hRes[(int64_t)row * (N * N) + (jj - 2 * N)] = rr + bias2;
+                        a->hRes[(int64_t)row * (N * N) + (jj - 2 * N)] = rr + bias2;
                     }
                 }
             }
@@ -562,10 +566,10 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     __shared__ uint32_t epochSh;
 
     const int tid = threadIdx.x;
-    // Thread 0 reads the epoch the previous launch on this workspace left; the
-    // load is waited for only where the epoch is first needed.
-    const uint32_t prevEpoch = tid == 0 ? epoch_load(a.hdr, kWsEpochOff) : 0u;
+    // (A captured launch's load is waited for only where the epoch is first
+    // needed.)
     const int g = blockIdx.x;
+    const uint32_t replays = tid == 0 ? replay_load(a.tag.words, g) : 0u;
     const int xcd = g % a.nXcd;
     const int j = g / a.nXcd;
     const int teamSize = a.P + a.R;
@@ -573,7 +577,7 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     if (tj >= a.teamsPerXcd) {
         // Spare workgroup: the whole workgroup leaves together.
         if (tid == 0) {
-            epoch_mark(a.hdr, kWsSeenOff, epoch_next(prevEpoch), g);
+            (void)launch_epoch<StripArgs>(g, replays);
         }
         return;
     }
@@ -599,13 +603,13 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
         float *lds = &part[0][0][0][0];
         const int rr = role - a.P;
         if (a.P <= 8) {
-            reducer_wg<N, 8, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, 8, kBf16, kOwn>(team, (int)ntiles, rr, a.R, local, lds, replays, &epochSh);
         } else if (a.P <= 16) {
-            reducer_wg<N, 16, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, 16, kBf16, kOwn>(team, (int)ntiles, rr, a.R, local, lds, replays, &epochSh);
         } else if (a.P <= 32) {
-            reducer_wg<N, 32, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, 32, kBf16, kOwn>(team, (int)ntiles, rr, a.R, local, lds, replays, &epochSh);
         } else {
-            reducer_wg<N, kMaxSlices, kBf16, kOwn>(a, team, (int)ntiles, rr, a.R, local, lds, prevEpoch, &epochSh);
+            reducer_wg<N, kMaxSlices, kBf16, kOwn>(team, (int)ntiles, rr, a.R, local, lds, replays, &epochSh);
         }
         return;
     }
@@ -640,7 +644,7 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     }
     if (ntiles == 0) {
         if (tid == 0) {
-            epoch_mark(a.hdr, kWsSeenOff, epoch_next(prevEpoch), g);
+            (void)launch_epoch<StripArgs>(g, replays);
         }
         return;
     }
@@ -861,8 +865,7 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
         }
     }
     if (tid == 0) {
-        epochSh = epoch_next(prevEpoch);
-        epoch_mark(a.hdr, kWsSeenOff, epochSh, g);
+        epochSh = launch_epoch<StripArgs>(g, replays);
     }
     lds_barrier();
     const uint32_t epoch = __builtin_amdgcn_readfirstlane(epochSh);
@@ -1209,15 +1212,6 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     } else if (timedOut && lane == 0) {
         st_status_word(a.statusWord);
     }
-    // Workgroup 0 (always a slice workgroup of team 0) advances the
-    // workspace's epoch once every workgroup has taken this one.
-    if (g == 0 && w == 0) {
-        if (!epoch_publish(a.hdr, kWsEpochOff, kWsSeenOff, epoch, (int)gridDim.x, kOwn ? kPublishPolls : spinLimit) &&
-            !kOwn && lane == 0) {
-            st_status(statusW, launchId);
-            st_status_word(a.statusWord);
-        }
-    }
 }
 
 template <int N, bool kBf16, bool kPrep, bool kOwn>
@@ -1233,7 +1227,8 @@ int strip_coresident_t(int numCUs)
 }
 
 template <int N, bool kBf16, bool kPrep, bool kOwn>
-hipError_t launch_strip_t(const Plan &p, void *workspace, uint32_t launchId, hipStream_t stream)
+hipError_t launch_strip_t(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId,
+                          hipStream_t stream)
 {
     char *ws = static_cast<char *>(workspace);
     StripArgs a;
@@ -1248,6 +1243,7 @@ hipError_t launch_strip_t(const Plan &p, void *workspace, uint32_t launchId, hip
     a.hRes = p.hRes;
     a.hPre = p.hasHPre ? p.hPre : nullptr;
     a.hdr = ws;
+    a.tag = tag;
     a.statusWord = p.statusWord;
     a.bcast = reinterpret_cast<uint64_t *>(ws + p.wsStripBcast);
     a.recs = reinterpret_cast<uint64_t *>(ws + p.wsStripRecs);
@@ -1295,14 +1291,15 @@ auto strip_instance(const Plan &p, F &&f)
 }
 }  // namespace
 
-hipError_t launch_strip(const Plan &p, void *workspace, uint32_t launchId, hipStream_t stream)
+hipError_t launch_strip(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId,
+                          hipStream_t stream)
 {
     if (p.n != 4) {
         return hipErrorNotSupported;
     }
     return strip_instance(p, [&](auto bf16, auto prep, auto own) {
-        return launch_strip_t<4, decltype(bf16)::value, decltype(prep)::value, decltype(own)::value>(p, workspace,
-                                                                                                    launchId, stream);
+        return launch_strip_t<4, decltype(bf16)::value, decltype(prep)::value, decltype(own)::value>(
+            p, workspace, tag, launchId, stream);
     });
 }
 
