@@ -270,8 +270,15 @@ MHC_API const char *mhcPreStatusString(int status);
  * writes a static NUL-terminated name to *name.  The name is that of the
  * path the shape belongs to: small batches run the cell kernel, "rows" and
  * "split" shapes with n = 6 the slab kernel, and "split" shapes with n = 4 the
- * strip kernel, instead of the path's own kernels where that is faster. */
+ * strip kernel, instead of the path's own kernels where that is faster
+ * (mhcPreExecutorKernel tells which one ran). */
 MHC_API int mhcPreExecutorPath(const mhcPreExecutor *executor, const char **name);
+
+/* Which kernel the executor's latest launch ran, "cell", "slab", "strip",
+ * "fused", "rows" or "split" (before the first launch: the one it is planned
+ * for, which a device that cannot hold its grid replaces by the path's own).
+ * Diagnostics and tests; no counterpart in the reference. */
+MHC_API int mhcPreExecutorKernel(const mhcPreExecutor *executor, const char **name);
 
 /*
  * Measurement aid, no counterpart in the reference: enqueues one launch of a

@@ -92,6 +92,8 @@ def load_library() -> ctypes.CDLL:
     lib.mhcPreStatusString.restype = ctypes.c_char_p
     lib.mhcPreExecutorPath.argtypes = [exe, P(ctypes.c_char_p)]
     lib.mhcPreExecutorPath.restype = ctypes.c_int
+    lib.mhcPreExecutorKernel.argtypes = [exe, P(ctypes.c_char_p)]
+    lib.mhcPreExecutorKernel.restype = ctypes.c_int
     lib.mhcPreNoAlloc.argtypes = [exe, ctypes.c_void_p]
     lib.mhcPreNoAlloc.restype = ctypes.c_int
     lib.mhcPreExecutorSetStatusWord.argtypes = [exe, ctypes.c_void_p]
@@ -306,6 +308,16 @@ class MhcPreOp:
         st = self.lib.mhcPreExecutorPath(self.executor, ctypes.byref(name))
         if st != 0:
             raise MhcPreError("mhcPreExecutorPath", st)
+        return name.value.decode()
+
+    @property
+    def kernel(self) -> str:
+        """The kernel that the latest launch ran, or that the first one is
+        planned for (mhcPreExecutorKernel)."""
+        name = ctypes.c_char_p()
+        st = self.lib.mhcPreExecutorKernel(self.executor, ctypes.byref(name))
+        if st != 0:
+            raise MhcPreError("mhcPreExecutorKernel", st)
         return name.value.decode()
 
     def launch(self, stream=None, check: bool = False) -> None:

@@ -86,6 +86,8 @@ struct mhcPreExecutor {
     // Host id of this executor's latest launch; the device status word only
     // reports a timeout written under it.
     std::atomic<uint32_t> lastLaunchId{0};
+    // Name of the kernel that launch ran (static storage); null before it.
+    std::atomic<const char *> lastKernel{nullptr};
     // Workgroups of the strip / fused kernel the device holds at once
     // (occupancy query, made once per executor: at phase 1 when the current
     // device holds x, else at the first launch); -2 until known.
@@ -1120,12 +1122,14 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     const uint32_t launchId = next_launch_id();
     executor->lastLaunchId.store(launchId, std::memory_order_relaxed);
     mhc::LaunchTag tag;
+    const char *kernel = "split";
     if (p.cellP > 0 && p.cellGrid <= mhc::kMaxExchangeGrid &&
         cached_coresident(executor->cellCoresident, mhc::cell_max_coresident, p, shape.cus) >= p.cellGrid) {
         err = mhc::make_launch_tag(launchId, device, p.cellGrid, workspace, stream, tag);
         if (err == hipSuccess) {
             err = mhc::launch_cell(p, workspace, tag, stream);
         }
+        kernel = "cell";
         done = true;
     }
     if (!done && (p.path == mhc::Path::kStrip || p.stripInstead)) {
@@ -1157,6 +1161,7 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
             if (err == hipSuccess) {
                 err = mhc::launch_strip(lp, workspace, tag, launchId, stream);
             }
+            kernel = "strip";
             done = true;
         }
     }
@@ -1182,6 +1187,7 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
             if (err == hipSuccess) {
                 err = mhc::launch_fused(lp, workspace, tag, launchId, stream);
             }
+            kernel = "fused";
             done = true;
         }
     }
@@ -1191,10 +1197,12 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
         if (err == hipSuccess) {
             err = mhc::launch_slab(p, workspace, tag, stream);
         }
+        kernel = "slab";
         done = true;
     }
     if (!done && p.path == mhc::Path::kRows) {
         err = mhc::launch_rows(p, workspace, shape.xcds, stream);
+        kernel = "rows";
         done = true;
     }
     if (!done) {
@@ -1203,6 +1211,7 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
         }
         err = mhc::launch_split(p, workspace, stream);
     }
+    executor->lastKernel.store(kernel, std::memory_order_relaxed);
     return err == hipSuccess ? MHC_STATUS_SUCCESS : MHC_STATUS_HIP_ERROR;
 }
 
@@ -1574,6 +1583,23 @@ int mhcPreExecutorPath(const mhcPreExecutor *executor, const char **name)
         break;
     }
     return MHC_STATUS_SUCCESS;
+}
+
+int mhcPreExecutorKernel(const mhcPreExecutor *executor, const char **name)
+{
+    if (executor == nullptr || name == nullptr) {
+        return MHC_STATUS_NULL_ARGUMENT;
+    }
+    *name = executor->lastKernel.load(std::memory_order_relaxed);
+    if (*name != nullptr) {
+        return MHC_STATUS_SUCCESS;
+    }
+    const mhc::Plan &p = executor->plan;
+    if (p.cellP > 0 || p.stripInstead || p.slab.P > 0) {
+        *name = p.cellP > 0 ? "cell" : p.stripInstead ? "strip" : "slab";
+        return MHC_STATUS_SUCCESS;
+    }
+    return mhcPreExecutorPath(executor, name);
 }
 
 int mhcPreStreamProbe(const void *src, uint64_t readBytes, void *dst, uint64_t writeBytes,

@@ -25,25 +25,26 @@ def _inputs(n, T, D, is_bf16, has_gamma):
     return to_bits(xf, is_bf16), phi, alpha, bias, gamma
 
 
-@pytest.mark.parametrize("n,T,D,is_bf16,has_gamma,path", [
-    (4, 1, 16, True, True, "split"),       # one slice, a quarter of a strip
-    (4, 33, 256, False, False, "rows"),    # 4 narrow slices, three row tiles
-    (4, 512, 1024, True, True, "strip"),   # the largest grid: two workgroups per CU
-    (4, 17, 8192, False, True, "rows"),    # 64 slices
-    (4, 100, 1200, True, False, "split"),  # D % 64 == 48, wide slices
-    (6, 5, 80, True, True, "split"),       # streams that start in mid k-step
-    (6, 130, 2560, False, True, "rows"),   # more workgroups than are resident: the path's kernels
-    (6, 112, 2560, True, True, "rows"),    # two workgroups per CU
-    (6, 31, 7168, True, False, "rows"),
-    (8, 16, 16, False, True, "rows"),
-    (8, 250, 496, True, True, "rows"),
-    (8, 9, 3056, True, False, "rows"),     # wide slices, the last 112 columns
+@pytest.mark.parametrize("n,T,D,is_bf16,has_gamma,path,kernel", [
+    (4, 1, 16, True, True, "split", "cell"),       # one slice, a quarter of a strip
+    (4, 33, 256, False, False, "rows", "cell"),    # 4 narrow slices, three row tiles
+    (4, 512, 1024, True, True, "strip", "cell"),   # the largest grid: two workgroups per CU
+    (4, 17, 8192, False, True, "rows", "cell"),    # 64 slices
+    (4, 100, 1200, True, False, "split", "cell"),  # D % 64 == 48, wide slices
+    (6, 5, 80, True, True, "split", "cell"),       # streams that start in mid k-step
+    (6, 130, 2560, False, True, "rows", "rows"),   # more workgroups than are resident: the path's kernels
+    (6, 112, 2560, True, True, "rows", "cell"),    # two workgroups per CU
+    (6, 31, 7168, True, False, "rows", "cell"),
+    (8, 16, 16, False, True, "rows", "cell"),
+    (8, 250, 496, True, True, "rows", "cell"),
+    (8, 9, 3056, True, False, "rows", "cell"),     # wide slices, the last 112 columns
 ])
-def test_cell(pkg, orc, device, n, T, D, is_bf16, has_gamma, path):
+def test_cell(pkg, orc, device, n, T, D, is_bf16, has_gamma, path, kernel):
     x, phi, alpha, bias, gamma = _inputs(n, T, D, is_bf16, has_gamma)
     _say(f"[cell] n={n} T={T} D={D} bf16={is_bf16} gamma={has_gamma}")
     ref = orc.mhc_pre(x, is_bf16, phi, alpha, bias, gamma)
-    plain = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="cell")
+    plain = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="cell",
+                    kernel=kernel)
     os.environ["MHCPRE_FORCE_PATH"] = "cell"
     try:
         xt, pt, at, bt, gt = to_device(pkg, device, x, is_bf16, phi, alpha, bias, gamma)
@@ -53,6 +54,7 @@ def test_cell(pkg, orc, device, n, T, D, is_bf16, has_gamma, path):
     assert plain.pop("path") == path
     check(plain, ref, x, is_bf16, orc)
     op.launch(check=True)  # prepared weights: the same bits
+    assert op.kernel == kernel
     got = fetch(op)
     for k in plain:
         assert np.array_equal(got[k], plain[k]), k
@@ -80,6 +82,7 @@ def test_expired_waits_are_computed(pkg, orc, device, n, T, D, prepared):
             t.fill_(float("nan"))
         _say(f"[cell] n={n} T={T} D={D} spin limit 0")
         op.launch(check=True)
+        assert op.kernel == "cell"
         got = fetch(op)
         for k in got:
             assert np.array_equal(got[k], want[k]), k
@@ -107,4 +110,5 @@ def test_graph_replays_on_new_inputs(pkg, orc, device):
         torch.cuda.synchronize()
         check(fetch(op), orc.mhc_pre(xr, True, phi, alpha, bias, gamma), xr, True, orc)
         op.launch(check=True)
+        assert op.kernel == "cell"
     op.close()

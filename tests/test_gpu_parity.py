@@ -35,7 +35,7 @@ def to_device(pkg, device, x_bits, is_bf16, phi, alpha, bias, gamma, lead=None):
 
 
 def run_gpu(pkg, device, x_bits, is_bf16, phi, alpha, bias, gamma, norm_eps=1e-6, hc_eps=1e-6,
-            lead=None, h_pre=True, force_path=None, launch=None):
+            lead=None, h_pre=True, force_path=None, launch=None, kernel=None):
     import os
 
     import torch
@@ -54,6 +54,7 @@ def run_gpu(pkg, device, x_bits, is_bf16, phi, alpha, bias, gamma, norm_eps=1e-6
     op.launch()
     torch.cuda.synchronize()
     assert op.device_status() == 0
+    assert kernel is None or op.kernel == kernel
     out = fetch(op)
     out["path"] = op.path
     op.close()

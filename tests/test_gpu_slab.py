@@ -40,7 +40,7 @@ def _inputs(T, D, is_bf16, has_gamma, seed=0):
 def test_slab_shapes(pkg, orc, device, T, D, is_bf16, has_gamma):
     x, phi, alpha, bias, gamma = _inputs(T, D, is_bf16, has_gamma)
     _say(f"[slab] T={T} D={D} bf16={is_bf16} gamma={has_gamma}")
-    out = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="slab")
+    out = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="slab", kernel="slab")
     check(out, orc.mhc_pre(x, is_bf16, phi, alpha, bias, gamma), x, is_bf16, orc)
 
 
@@ -51,10 +51,10 @@ def test_slab_geometries_agree(pkg, orc, device, geometry):
     gives the same bits."""
     T, D = 1500, 1024
     x, phi, alpha, bias, gamma = _inputs(T, D, True, True)
-    want = run_gpu(pkg, device, x, True, phi, alpha, bias, gamma, force_path="slab")
+    want = run_gpu(pkg, device, x, True, phi, alpha, bias, gamma, force_path="slab", kernel="slab")
     os.environ["MHCPRE_SLAB"] = geometry
     try:
-        got = run_gpu(pkg, device, x, True, phi, alpha, bias, gamma, force_path="slab")
+        got = run_gpu(pkg, device, x, True, phi, alpha, bias, gamma, force_path="slab", kernel="slab")
     finally:
         os.environ.pop("MHCPRE_SLAB", None)
     check(got, orc.mhc_pre(x, True, phi, alpha, bias, gamma), x, True, orc)
@@ -75,6 +75,7 @@ def test_slab_prepared_matches_plain(pkg, orc, device, T, D, is_bf16):
         os.environ.pop("MHCPRE_FORCE_PATH", None)
     plain.launch(check=True)
     prep.launch(check=True)
+    assert plain.kernel == "slab" and prep.kernel == "slab"
     a, b = fetch(plain), fetch(prep)
     check(a, orc.mhc_pre(x, is_bf16, phi, alpha, bias, gamma), x, is_bf16, orc)
     for k in a:
@@ -107,6 +108,7 @@ def test_slab_expired_waits_are_computed(pkg, orc, device, T, D, prepared):
             t.fill_(float("nan"))
         _say(f"[slab] T={T} D={D} {'calm' if op is calm else 'spin limit 0'}")
         op.launch(check=True)
+        assert op.kernel == "slab"
         check(fetch(op), ref, x, True, orc)
     hurried.close()
     calm.close()
@@ -131,6 +133,7 @@ def test_slab_graph_replays(pkg, orc, device):
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
+        assert op.kernel == "slab"
         replayed = fetch(op)
         check(replayed, orc.mhc_pre(xs[i], True, phi, alpha, bias, gamma), xs[i], True, orc)
         op.launch(check=True)

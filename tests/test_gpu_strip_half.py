@@ -40,7 +40,8 @@ def test_strip_at_half_step_widths(pkg, orc, device, T, D, is_bf16, has_gamma, p
     x, phi, alpha, bias, gamma = _inputs(T, D, is_bf16, has_gamma)
     _say(f"[strip half] T={T} D={D} bf16={is_bf16} gamma={has_gamma} prepared={prepared}")
     ref = orc.mhc_pre(x, is_bf16, phi, alpha, bias, gamma)
-    plain = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="strip")
+    plain = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="strip",
+                    kernel="strip")
     os.environ["MHCPRE_FORCE_PATH"] = "strip"
     try:
         xt, pt, at, bt, gt = to_device(pkg, device, x, is_bf16, phi, alpha, bias, gamma)
@@ -51,6 +52,7 @@ def test_strip_at_half_step_widths(pkg, orc, device, T, D, is_bf16, has_gamma, p
     check(plain, ref, x, is_bf16, orc)
     if prepared:  # the same bits from prepared weights
         op.launch(check=True)
+        assert op.kernel == "strip"
         got = fetch(op)
         for k in plain:
             assert np.array_equal(got[k], plain[k]), k
@@ -79,5 +81,6 @@ def test_expired_waits_are_computed(pkg, orc, device, T, D, prepared):
             t.fill_(float("nan"))
         _say(f"[strip half] T={T} D={D} spin limit 0")
         op.launch(check=True)
+        assert op.kernel == "strip"
         check(fetch(op), ref, x, True, orc)
     op.close()
