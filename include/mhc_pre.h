@@ -150,8 +150,9 @@ MHC_API int mhcPreGetWorkspaceSizeWithHPre(const mhcTensor *x, const mhcTensor *
  *
  * The cell kernel (small batches), the slab kernel (n = 6) and the strip kernel
  * at D % 32 == 16 wait between workgroups in the same way, but a workgroup whose
- * wait expires computes what it waited for itself: such a launch is slow and
- * its outputs are right, so nothing is reported.
+ * wait expires computes what it waited for itself, in the order of the exchange:
+ * such a launch is slow and its outputs have the same bits, so it is no error
+ * (mhcPreQueryComputedWaits tells).
  *
  * A launch may be captured into a HIP graph and replayed.  What tells the
  * current launch's exchange data from everything the workspace held before is
@@ -279,6 +280,17 @@ MHC_API int mhcPreExecutorPath(const mhcPreExecutor *executor, const char **name
  * for, which a device that cannot hold its grid replaces by the path's own).
  * Diagnostics and tests; no counterpart in the reference. */
 MHC_API int mhcPreExecutorKernel(const mhcPreExecutor *executor, const char **name);
+
+/*
+ * Writes 1 to *computed if a workgroup of this executor's latest launch on
+ * `workspace` computed what an expired wait was for (the cell and slab kernels,
+ * the strip kernel at D % 32 == 16: the outputs are right, the launch was slow
+ * because other work held the CUs it needs), else 0.  Synchronizes `stream`
+ * first; workspace NULL with workspaceSize 0 as in mhcPreQueryDeviceStatus.
+ * Diagnostics and tests; no counterpart in the reference.
+ */
+MHC_API int mhcPreQueryComputedWaits(void *workspace, uint64_t workspaceSize, const mhcPreExecutor *executor,
+                                     hipStream_t stream, int32_t *computed);
 
 /*
  * Measurement aid, no counterpart in the reference: enqueues one launch of a

@@ -94,6 +94,9 @@ def load_library() -> ctypes.CDLL:
     lib.mhcPreExecutorPath.restype = ctypes.c_int
     lib.mhcPreExecutorKernel.argtypes = [exe, P(ctypes.c_char_p)]
     lib.mhcPreExecutorKernel.restype = ctypes.c_int
+    lib.mhcPreQueryComputedWaits.argtypes = [ctypes.c_void_p, ctypes.c_uint64, exe,
+                                             ctypes.c_void_p, P(ctypes.c_int32)]
+    lib.mhcPreQueryComputedWaits.restype = ctypes.c_int
     lib.mhcPreNoAlloc.argtypes = [exe, ctypes.c_void_p]
     lib.mhcPreNoAlloc.restype = ctypes.c_int
     lib.mhcPreExecutorSetStatusWord.argtypes = [exe, ctypes.c_void_p]
@@ -385,6 +388,19 @@ class MhcPreOp:
                                                 ctypes.c_uint64(self.workspace_size),
                                                 self.executor,
                                                 ctypes.c_void_p(_stream_handle(stream)))
+
+    def computed_waits(self, stream=None) -> bool:
+        """Synchronize ``stream``; whether the latest launch on this object's
+        workspace computed what an expired wait was for
+        (mhcPreQueryComputedWaits)."""
+        out = ctypes.c_int32(0)
+        st = self.lib.mhcPreQueryComputedWaits(ctypes.c_void_p(self.workspace.data_ptr()),
+                                               ctypes.c_uint64(self.workspace_size), self.executor,
+                                               ctypes.c_void_p(_stream_handle(stream)),
+                                               ctypes.byref(out))
+        if st != 0:
+            raise MhcPreError("mhcPreQueryComputedWaits", st)
+        return bool(out.value)
 
     def close(self) -> None:
         if getattr(self, "executor", None) is not None and self.executor.value:

@@ -363,7 +363,8 @@ bool slab_faster(int64_t D, int64_t T)
 }
 
 // Phase-1 knobs for tests and measurement sweeps (MHCPRE_FORCE_PATH,
-// MHCPRE_SPIN_LIMIT, MHCPRE_ROWS_B, MHCPRE_ROWS_PARTIALS, MHCPRE_SLAB, MHCPRE_CELL) are read only when
+// MHCPRE_SPIN_LIMIT, MHCPRE_SPIN_EVERY, MHCPRE_ROWS_B, MHCPRE_ROWS_PARTIALS,
+// MHCPRE_SLAB, MHCPRE_CELL; MHCPRE_REPLAY_WORDS at a capture) are read only when
 // MHCPRE_TESTING=1: a stray one in a production environment changes nothing.
 const char *test_env(const char *name)
 {
@@ -866,6 +867,9 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
     if (const char *launch = std::getenv("MHCPRE_LAUNCH")) {
         p.fusedCooperative = std::strcmp(launch, "cooperative") == 0;
     }
+    if (const char *every = test_env("MHCPRE_SPIN_EVERY")) {
+        p.spinEvery = static_cast<uint32_t>(std::strtoul(every, nullptr, 10));
+    }
     if (const char *spin = test_env("MHCPRE_SPIN_LIMIT")) {
         char *end = nullptr;
         const unsigned long v = std::strtoul(spin, &end, 10);
@@ -956,10 +960,19 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
                                                                     mhc::cell_record_bytes(),
                                                                 256));
     }
+    // The strips over all of K that a wave's share of the tiles takes alone.
+    const auto own_strips = [&](int64_t teams, int groups, int64_t strips) {
+        const int64_t tiles = (rowTiles + teams - 1) / teams;
+        return (tiles + groups - 1) / groups * strips;
+    };
     if (p.stripInstead) {
-        if (p.stripMaxTeams < 1 || (stripEnd > mhc::kScratchBytes && p.wsTotal <= mhc::kScratchBytes)) {
+        const int64_t own = own_strips(std::max(p.stripMaxTeams, 1), mhc::strip_groups(),
+                                       int64_t{p.stripP} * mhc::strip_strips());
+        if (p.stripMaxTeams < 1 || own > mhc::kMaxOwnStrips ||
+            (stripEnd > mhc::kScratchBytes && p.wsTotal <= mhc::kScratchBytes)) {
             p.stripInstead = false;
         } else {
+            p.ownStrips = static_cast<int>(own);
             p.wsTotal = std::max(p.wsTotal, stripEnd);
         }
     }
@@ -975,9 +988,12 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
             align_up(p.wsSlabRecs + slots * p.slab.P * mhc::slab_record_words() * 8, 256);
         // Not where it would take a call past the built-in scratch that the
         // other kernels' layout fits.
-        if (slabEnd > mhc::kScratchBytes && p.wsTotal <= mhc::kScratchBytes) {
+        const int64_t own = own_strips(int64_t{p.slab.groups} * p.slab.teams, mhc::slab_groups(),
+                                       int64_t{p.slab.P} * mhc::slab_strips());
+        if (own > mhc::kMaxOwnStrips || (slabEnd > mhc::kScratchBytes && p.wsTotal <= mhc::kScratchBytes)) {
             p.slab = mhc::SlabGeometry{};
         } else {
+            p.ownStrips = static_cast<int>(own);
             p.wsTotal = std::max(p.wsTotal, slabEnd);
         }
     }
@@ -1127,7 +1143,7 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
         cached_coresident(executor->cellCoresident, mhc::cell_max_coresident, p, shape.cus) >= p.cellGrid) {
         err = mhc::make_launch_tag(launchId, device, p.cellGrid, workspace, stream, tag);
         if (err == hipSuccess) {
-            err = mhc::launch_cell(p, workspace, tag, stream);
+            err = mhc::launch_cell(p, workspace, tag, launchId, stream);
         }
         kernel = "cell";
         done = true;
@@ -1195,7 +1211,7 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
         cached_coresident(executor->slabCoresident, mhc::slab_max_coresident, p, shape.cus) >= shape.cus) {
         err = mhc::make_launch_tag(launchId, device, p.slab.grid, workspace, stream, tag);
         if (err == hipSuccess) {
-            err = mhc::launch_slab(p, workspace, tag, stream);
+            err = mhc::launch_slab(p, workspace, tag, launchId, stream);
         }
         kernel = "slab";
         done = true;
@@ -1213,6 +1229,36 @@ int launch_on(void *workspace, mhcPreExecutor *executor, hipStream_t stream)
     }
     executor->lastKernel.store(kernel, std::memory_order_relaxed);
     return err == hipSuccess ? MHC_STATUS_SUCCESS : MHC_STATUS_HIP_ERROR;
+}
+
+// The status word of `workspace` (null with size 0: the current device's
+// built-in one) after the stream's work, 0 unless the executor's latest launch
+// wrote it.
+int read_status_code(void *workspace, uint64_t workspaceSize, const mhcPreExecutor *executor, hipStream_t stream,
+                     uint32_t &code)
+{
+    if (workspace == nullptr && workspaceSize == 0) {
+        // The launches of mhcPreNoAlloc: the current device's built-in array.
+        int device = -1;
+        if (hipGetDevice(&device) != hipSuccess || mhc::scratch_address(device, &workspace) != hipSuccess) {
+            (void)hipGetLastError();
+            return MHC_STATUS_HIP_ERROR;
+        }
+        workspaceSize = mhc::kScratchBytes;
+    }
+    if (workspace == nullptr || workspaceSize < executor->plan.wsTotal) {
+        return MHC_STATUS_WORKSPACE_TOO_SMALL;
+    }
+    if (hipStreamSynchronize(stream) != hipSuccess) {
+        return MHC_STATUS_HIP_ERROR;
+    }
+    uint64_t word = 0;
+    if (hipMemcpy(&word, workspace, sizeof(word), hipMemcpyDeviceToHost) != hipSuccess) {
+        return MHC_STATUS_HIP_ERROR;
+    }
+    const bool own = static_cast<uint32_t>(word >> 32) == executor->lastLaunchId.load(std::memory_order_relaxed);
+    code = own ? static_cast<uint32_t>(word) : 0u;
+    return MHC_STATUS_SUCCESS;
 }
 
 // The occupancy queries of a new executor and the addresses of the device's
@@ -1507,30 +1553,12 @@ int mhcPreQueryDeviceStatus(void *workspace, uint64_t workspaceSize,
     if (executor == nullptr) {
         return MHC_STATUS_NULL_ARGUMENT;
     }
-    if (workspace == nullptr && workspaceSize == 0) {
-        // The launches of mhcPreNoAlloc: the current device's built-in array.
-        int device = -1;
-        if (hipGetDevice(&device) != hipSuccess || mhc::scratch_address(device, &workspace) != hipSuccess) {
-            (void)hipGetLastError();
-            return MHC_STATUS_HIP_ERROR;
-        }
-        workspaceSize = mhc::kScratchBytes;
+    uint32_t code = 0;
+    const int st = read_status_code(workspace, workspaceSize, executor, stream, code);
+    if (st != MHC_STATUS_SUCCESS) {
+        return st;
     }
-    if (workspace == nullptr || workspaceSize < executor->plan.wsTotal) {
-        return MHC_STATUS_WORKSPACE_TOO_SMALL;
-    }
-    if (hipStreamSynchronize(stream) != hipSuccess) {
-        return MHC_STATUS_HIP_ERROR;
-    }
-    uint64_t word = 0;
-    if (hipMemcpy(&word, workspace, sizeof(word), hipMemcpyDeviceToHost) != hipSuccess) {
-        return MHC_STATUS_HIP_ERROR;
-    }
-    const uint32_t code = static_cast<uint32_t>(word);
-    const uint32_t epoch = static_cast<uint32_t>(word >> 32);
-    const bool timedOut = code == mhc::kDeviceTimeout &&
-                          epoch == executor->lastLaunchId.load(std::memory_order_relaxed);
-    return timedOut ? MHC_STATUS_DEVICE_TIMEOUT : MHC_STATUS_SUCCESS;
+    return code == mhc::kDeviceTimeout ? MHC_STATUS_DEVICE_TIMEOUT : MHC_STATUS_SUCCESS;
 }
 
 const char *mhcPreStatusString(int status)
@@ -1600,6 +1628,20 @@ int mhcPreExecutorKernel(const mhcPreExecutor *executor, const char **name)
         return MHC_STATUS_SUCCESS;
     }
     return mhcPreExecutorPath(executor, name);
+}
+
+int mhcPreQueryComputedWaits(void *workspace, uint64_t workspaceSize, const mhcPreExecutor *executor,
+                             hipStream_t stream, int32_t *computed)
+{
+    if (executor == nullptr || computed == nullptr) {
+        return MHC_STATUS_NULL_ARGUMENT;
+    }
+    uint32_t code = 0;
+    const int st = read_status_code(workspace, workspaceSize, executor, stream, code);
+    if (st == MHC_STATUS_SUCCESS) {
+        *computed = code == mhc::kDeviceComputed ? 1 : 0;
+    }
+    return st;
 }
 
 int mhcPreStreamProbe(const void *src, uint64_t readBytes, void *dst, uint64_t writeBytes,

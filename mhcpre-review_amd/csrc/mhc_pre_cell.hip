@@ -80,6 +80,8 @@ struct CellArgs {
     float *hPre;
     uint64_t *recs;  // [column tile][row tile][P] records
     LaunchTag tag;
+    char *hdr;  // workspace header: the status word
+    uint32_t launchId;
     int T;
     int D;
     int K;
@@ -88,6 +90,7 @@ struct CellArgs {
     float hcEps;
     float invFlatDim;
     uint32_t spinLimit;
+    uint32_t spinEvery;
 };
 
 __device__ __forceinline__ uint32_t rec_tag(uint32_t pos, uint32_t epoch) { return (pos * 0x9E3779B1u) ^ epoch; }
@@ -357,8 +360,12 @@ __global__ __launch_bounds__((Cell<N, NS>::kThreads), (Cell<N, NS>::kWavesPerSim
         lds_barrier();
         expired = expiredSh != 0;
     }
-    if (expired) {
+    if (expired || hurried(a.spinEvery, group * P + p)) {
         // Every slice's sums once more, added in the same order: the same bits.
+        if (tid == 0) {
+            const auto *la = late_args<CellArgs>();
+            st_computed(la->hdr, la->launchId);
+        }
         float2 sum = make_float2(0.f, 0.f);
 #pragma unroll 1
         for (int g = 0; g < groups; ++g) {
@@ -461,7 +468,7 @@ struct Instance {
         }
         return perCU * numCUs;
     }
-    static hipError_t launch(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
+    static hipError_t launch(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream)
     {
         char *ws = static_cast<char *>(workspace);
         CellArgs a;
@@ -477,6 +484,8 @@ struct Instance {
         a.hPre = p.hasHPre ? p.hPre : nullptr;
         a.recs = reinterpret_cast<uint64_t *>(ws + p.wsCellRecs);
         a.tag = tag;
+        a.hdr = ws;
+        a.launchId = launchId;
         a.T = (int)p.T;
         a.D = (int)p.D;
         a.K = (int)p.K;
@@ -485,6 +494,7 @@ struct Instance {
         a.hcEps = p.hcEps;
         a.invFlatDim = p.invFlatDim;
         a.spinLimit = p.cellSpinLimit();
+        a.spinEvery = p.spinEvery;
         const unsigned tiles = (unsigned)((p.T + 15) / 16);
         const dim3 grid((unsigned)p.cellP, tiles, (unsigned)(p.cellGrid / (p.cellP * tiles)));
         const dim3 block(Cell<N, NS>::kThreads);
@@ -525,9 +535,9 @@ int cell_max_coresident(const Plan &p, int numCUs)
     return with_instance(p, [&](auto i) { return decltype(i)::coresident(numCUs); });
 }
 
-hipError_t launch_cell(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
+hipError_t launch_cell(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream)
 {
-    return with_instance(p, [&](auto i) { return decltype(i)::launch(p, workspace, tag, stream); });
+    return with_instance(p, [&](auto i) { return decltype(i)::launch(p, workspace, tag, launchId, stream); });
 }
 
 }  // namespace mhc

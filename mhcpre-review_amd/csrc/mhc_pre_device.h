@@ -307,6 +307,16 @@ __device__ __forceinline__ uint32_t launch_epoch(int g, uint32_t loaded)
     return a->tag.seed ^ mix32(loaded + 1u);
 }
 
+// Whether workgroup g is one that gives up its waits at once (Plan::spinEvery).
+__device__ __forceinline__ bool hurried(uint32_t every, int g) { return every != 0u && (uint32_t)g % every == 0u; }
+
+// The status word's report of an expired wait whose work was done instead.
+__device__ __forceinline__ void st_computed(void *hdr, uint32_t launchId)
+{
+    typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{kDeviceComputed, launchId}, make_rsrc(hdr, 8), 0, 0, kCpolDev);
+}
+
 // Quiet NaN written into the outputs of rows whose exchange wait expired.
 __device__ __forceinline__ float poison() { return __uint_as_float(0x7FC00000u); }
 
@@ -355,59 +365,202 @@ struct WeightsRef {
     int K;
 };
 
-// Sums of one row over all of K, by one wave (every lane gets them): mix
-// columns j0 .. j0 + 7 (0 past M) and the sum of squares; rows past T read
-// zeros.  For work whose exchange wait expired: any wave can do it alone.
-template <int N, bool kBf16>
-__device__ __forceinline__ void own_sums(const WeightsRef &wt, const uint16_t *x, int64_t T, int64_t row, int j0,
-                                         float (&acc)[9])
+// The lane, opaque: what is derived from it is derived where it is used, not
+// kept in registers from the start of the kernel.
+__device__ __forceinline__ int lane_here()
+{
+    int l = (int)(threadIdx.x & 63);
+    asm volatile("" : "+v"(l));
+    return l;
+}
+
+// What a launch whose exchange wait expired computes instead, by any wave alone
+// and in the order of the exchange, so that the outputs have the same bits.
+
+// One 64-column strip's sums of a 16-row tile: mix column j (every lane its
+// own; 0 from M on), in C fragments, and in lanes 16(r / 4) + r the sum of
+// squares of row r.  xr: the tile's valid rows; col0: the strip's first column.
+// kApart: hi and lo products in sums of their own, added at the end, and from
+// column 16 Q on fp16's x_lo meets both (the strip kernel; the slab kernel adds
+// all to one sum and x_lo meets hi only).
+template <int N, bool kBf16, bool kApart>
+__device__ __forceinline__ void strip_sums(const WeightsRef &wt, __amdgpu_buffer_rsrc_t xr, int D, int col0, int j,
+                                           f32x4_t &sum, float &sq)
 {
     constexpr int M = Shape<N>::M;
     constexpr int Q = M / 16;
+    const int lane = lane_here();
+    const int rl = lane & 15;
     const int K = wt.K;
     const bool prep = wt.bprep != nullptr;
     const bool hasGamma = wt.gamma != nullptr;
     const __amdgpu_buffer_rsrc_t pr = make_rsrc(wt.phi, prep ? 0 : M * K * 4);
     const __amdgpu_buffer_rsrc_t gr = make_rsrc(wt.gamma, hasGamma ? K * 4 : 0);
     const __amdgpu_buffer_rsrc_t br = make_rsrc(wt.bprep, prep ? M * K * 4 : 0);
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x + (row < T ? row : 0) * K, row < T ? K * 2 : 0);
+    // hi and lo of the prepared value (k, j): tiles j / 16 and Q + j / 16, or
+    // (j >= 16 Q) lanes j % 16 and + 8 of tile 2Q.
+    const bool half = j >= 16 * Q;
+    const int tile = half ? 2 * Q : j >> 4;
+    const int loOff = half ? 8 * 16 : Q * 64 * 16;
+    f32x4_t hiSum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t loSum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t gram = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int s = 0; s < N; ++s) {
 #pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        acc[i] = 0.f;
-    }
-#pragma unroll 1
-    for (int k = (int)(threadIdx.x & 63); k < K; k += 64) {
-        const float xv = x_to_f32<kBf16>((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(xr, 2 * k, 0, 0));
-        const float gv = hasGamma ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gr, 4 * k, 0, 0)) : 1.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int j = j0 + i;
-            float b;
+        for (int q = 0; q < 2; ++q) {
+            const int dc = col0 + 32 * q + 8 * (lane >> 4);
+            const int k = s * D + dc;
+            const bool live = dc < D;
+            const u32x4_t xf = load16<0>(xr, live ? (rl * K + k) * 2 : kPast);
+            u32x4_t hi, lo;
             if (prep) {
-                // hi + lo of the prepared fragments' value (k, j): tiles j / 16
-                // and Q + j / 16, or (j >= 16 Q) lanes j % 16 and + 8 of tile 2Q.
-                const bool half = j >= 16 * Q;
-                const int tile = half ? 2 * Q : j >> 4;
-                const int f = (((k >> 5) * Shape<N>::NT + tile) * 64 + 16 * ((k >> 3) & 3) + (j & 15)) * 16 + 2 * (k & 7);
-                const int off = j < M ? f : kPast;
-                b = bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, off, 0, 0)) +
-                    bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
-                        br, off + (half ? 8 * 16 : Q * 64 * 16), 0, 0));
+                const int f = (((k >> 5) * Shape<N>::NT + tile) * 64 + 16 * ((k >> 3) & 3) + (j & 15)) * 16;
+                const int off = live && j < M ? f : kPast;
+                hi = load16<0>(br, off);
+                lo = load16<0>(br, off + loOff);
             } else {
-                b = __uint_as_float(
-                        __builtin_amdgcn_raw_buffer_load_b32(pr, j < M ? (j * K + k) * 4 : kPast, 0, 0)) *
-                    gv;
+                const int off = live && j < M ? (j * K + k) * 4 : kPast;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const u32x4_t pv = load16<0>(pr, off + 16 * h);
+                    const u32x4_t gv = load16<0>(gr, live && hasGamma ? (k + 4 * h) * 4 : kPast);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        float a = __uint_as_float(pv[2 * e]);
+                        float c = __uint_as_float(pv[2 * e + 1]);
+                        if (hasGamma) {
+                            a = a * __uint_as_float(gv[2 * e]);
+                            c = c * __uint_as_float(gv[2 * e + 1]);
+                        }
+                        uint32_t hw, lw;
+                        split2_bf16(a, c, hw, lw);
+                        hi[2 * h + e] = hw;
+                        lo[2 * h + e] = lw;
+                    }
+                }
             }
-            acc[i] = __builtin_fmaf(xv, b, acc[i]);
+            u32x4_t xh = xf;
+            u32x4_t xl = u32x4_t{0u, 0u, 0u, 0u};
+            if constexpr (kBf16) {
+                gram = mfma16(xf, xf, gram);
+            } else {
+                gram = mfma16_f16(xf, xf, gram);
+                float f[8];
+                unpack8<false>(xf, f);
+                split_f16_to_bf16(f, xh, xl);
+            }
+            hiSum = mfma16(xh, hi, hiSum);
+            if constexpr (!kBf16) {
+                hiSum = mfma16(xl, hi, hiSum);
+            }
+            if constexpr (kApart) {
+                loSum = mfma16(xh, lo, loSum);
+                if constexpr (!kBf16) {
+                    const f32x4_t both = mfma16(xl, lo, loSum);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        loSum[e] = half ? both[e] : loSum[e];
+                    }
+                }
+            } else {
+                hiSum = mfma16(xh, lo, hiSum);
+            }
         }
-        acc[8] = __builtin_fmaf(xv, xv, acc[8]);
     }
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            acc[i] = acc[i] + __shfl_xor(acc[i], m);
+    sum = kApart ? hiSum + loSum : hiSum;
+    const int di = rl & 3;
+    sq = di == 0 ? gram[0] : di == 1 ? gram[1] : di == 2 ? gram[2] : gram[3];
+}
+
+// The sums of the slices g, g + G, ... of P, each of kStrips strips.
+template <int N, bool kBf16, bool kApart, int kStrips>
+__device__ __forceinline__ void group_sums(const WeightsRef &wt, __amdgpu_buffer_rsrc_t xr, int D, int P, int j,
+                                           int g, int G, f32x4_t &sum, float &sq)
+{
+    sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    sq = 0.f;
+#pragma unroll 1
+    for (int p = g; p < P; p += G) {
+        f32x4_t slice;
+        float sliceSq;
+#pragma unroll 1
+        for (int st = 0; st < kStrips; ++st) {
+            f32x4_t v;
+            float u;
+            strip_sums<N, kBf16, kApart>(wt, xr, D, 64 * (kStrips * p + st), j, v, u);
+            slice = st == 0 ? v : slice + v;
+            sliceSq = st == 0 ? u : sliceSq + u;
         }
+        sum = sum + slice;
+        sq = sq + sliceSq;
+    }
+}
+
+// The resource of the valid rows of tile rt of x.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const uint16_t *x, int64_t T, int K, int64_t rt)
+{
+    const int rows = (int)min((int64_t)16, T - 16 * rt);
+    return make_rsrc(x + 16 * rt * K, rows * K * 2);
+}
+
+// hIn of one wave's 64 columns from col0 of tile rt, with the tile's hPre from
+// all of its P slices, added in G groups.
+template <int N, bool kBf16, bool kApart, int kStrips>
+__device__ __forceinline__ void own_hin(const WeightsRef &wt, const uint16_t *x, uint16_t *hIn, const float *alpha,
+                                        const float *bias, int64_t T, int D, int64_t rt, int P, int G, int col0,
+                                        float invFlatDim, float normEps, float hcEps)
+{
+    const int lane = lane_here();
+    const int rl = lane & 15;
+    const int grp = lane >> 4;
+    const __amdgpu_buffer_rsrc_t xr = tile_rsrc(x, T, wt.K, rt);
+    f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float sq = 0.f;
+#pragma unroll 1
+    for (int g = 0; g < G; ++g) {
+        f32x4_t v;
+        float u;
+        group_sums<N, kBf16, kApart, kStrips>(wt, xr, D, P, rl, g, G, v, u);
+        sum = sum + v;
+        sq = sq + u;
+    }
+    f32x4_t pre;  // lane (stream, grp): rows 4 grp .. + 3
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float ir = ref_inv_rms(__shfl(sq, 20 * grp + e), invFlatDim, normEps);
+        pre[e] = ref_sigmoid(sum[e] * (ir * alpha[0]), bias[rl < N ? rl : 0], hcEps);
+    }
+    const int rows = (int)min((int64_t)16, T - 16 * rt);
+    const __amdgpu_buffer_rsrc_t hr = make_rsrc(hIn + 16 * rt * D, rows * D * 2);
+    const int col = col0 + 8 * grp + 32 * ((lane >> 3) & 1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int row = 8 * h + (lane & 7);
+        float hv[8];
+#pragma unroll
+        for (int s = 0; s < N; ++s) {
+            // Row `row` of stream s: lane 16 (row / 4) + s, element row % 4.
+            float pv = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = __shfl(pre[e], 16 * (row >> 2) + s);
+                pv = (row & 3) == e ? v : pv;
+            }
+            float f[8];
+            unpack8<kBf16>(load16<0>(xr, col < D ? (row * wt.K + s * D + col) * 2 : kPast), f);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float prod = pv * f[e];
+                hv[e] = s == 0 ? prod : hv[e] + prod;
+            }
+        }
+        u32x4_t out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            out[e] = pack2_x<kBf16>(hv[2 * e], hv[2 * e + 1]);
+        }
+        store16<0>(out, hr, col < D ? (row * D + col) * 2 : kPast);
     }
 }
 

@@ -18,9 +18,12 @@ enum class Path : int {
 // Device status word (first 8 bytes of the workspace): the low half holds a
 // code, the high half the host launch id of the launch that wrote it.  The
 // strip and fused kernels write (launch id, kDeviceTimeout) only when a wait
-// runs out; the split path's first kernel writes kDeviceOk into the low half.
+// runs out, kernels that then compute what they waited for (launch id,
+// kDeviceComputed); the split path's first kernel writes kDeviceOk into the low
+// half.
 constexpr uint32_t kDeviceOk = 0u;
 constexpr uint32_t kDeviceTimeout = 0x7107u;
+constexpr uint32_t kDeviceComputed = 0x7108u;  // an expired wait's work was done instead: the outputs are right
 
 // Bytes reserved at the head of the workspace: the status word at 0, and words
 // that only launches captured when the library's own were used up need
@@ -57,6 +60,10 @@ hipError_t make_launch_tag(uint32_t launchId, int device, int grid, void *worksp
                            LaunchTag &tag);
 // The current device's array of replay words (looked up once per device).
 hipError_t replay_words_address(int device, uint32_t **ptr);
+
+// The most that a wave may have to compute (Plan::ownStrips, about a second)
+// where the slab or strip kernel runs in place of kernels that wait for nobody.
+constexpr int64_t kMaxOwnStrips = int64_t{1} << 17;
 
 // Work distribution of the slab kernel (mhc_pre_slab.hip).
 struct SlabGeometry {
@@ -95,13 +102,27 @@ struct Plan {
     // gives up (about a second).  MHCPRE_SPIN_LIMIT at phase 1 overrides it,
     // for tests of the timeout path.
     uint32_t spinLimit = 1u << 20;
+    // Test knob (MHCPRE_SPIN_EVERY=k): in kernels whose expired waits are
+    // computed, every k-th workgroup gives up at its first poll (in the cell
+    // kernel also where that finds its data); 0: none.
+    uint32_t spinEvery = 0;
     // The same for kernels whose expired waits are computed instead: about as
-    // long as the computation takes, so that two such launches that hold half
-    // of each other's CUs do not stand still for a second (the cell kernel
-    // recomputes a row tile in up to 0.2 ms, the slab kernel and the strip
-    // kernel at D % 32 == 16 a workgroup's rows in some 20 ms).
-    uint32_t cellSpinLimit() const { return spinLimit < (1u << 9) ? spinLimit : 1u << 9; }
-    uint32_t ownSpinLimit() const { return spinLimit < (1u << 14) ? spinLimit : 1u << 14; }
+    // long as that takes, so that such a launch takes at most about twice as
+    // long as it had to (two launches that hold half of each other's CUs would
+    // stand still otherwise).  Measured on MI355X with every wait expired: the
+    // cell kernel 2 to 4 us per slice (n = 4, D = 1024, T = 512 38 us, n = 4, D =
+    // 7168, T = 16 126); a wave of the slab and strip kernels 6 to 10 us per
+    // 64-column strip of a tile's rows, over all of K (n = 6, D = 1024, T = 2048
+    // 0.36 ms, D = 4096, T = 4096 6.3 ms; n = 4, D = 7056, T = 2048 5.9 ms).  A
+    // poll takes about 0.7 us.  (At least 2^12 there: a first tile's hPre is
+    // waited for more than 64 polls in an undisturbed launch.)
+    uint32_t cellSpinLimit() const { return spinLimit < 64u + 4u * cellP ? spinLimit : 64u + 4u * cellP; }
+    uint32_t ownSpinLimit() const
+    {
+        const uint32_t polls = ownStrips < (1 << 9) ? 1u << 12 : 8u * (uint32_t)ownStrips;
+        return spinLimit < polls ? spinLimit : polls;
+    }
+    int ownStrips = 0;  // strips that a wave of the slab or strip kernel computes if its first wait expires
     float normEps = 1e-6f;
     float hcEps = 1e-6f;
     float invFlatDim = 0.f;  // fl(1.0f / K), as code/op_host/mhc_pre.cpp:154
@@ -210,16 +231,18 @@ hipError_t launch_fused(const Plan &plan, void *workspace, const LaunchTag &tag,
 hipError_t launch_strip(const Plan &plan, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream);
 
 // Cell kernel (mhc_pre_cell.hip).
-hipError_t launch_cell(const Plan &plan, void *workspace, const LaunchTag &tag, hipStream_t stream);
+hipError_t launch_cell(const Plan &plan, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream);
 int cell_max_coresident(const Plan &plan, int numCUs);
 size_t cell_record_bytes();
 
 // Slab kernel (mhc_pre_slab.hip): one launch, x read once.
-hipError_t launch_slab(const Plan &plan, void *workspace, const LaunchTag &tag, hipStream_t stream);
+hipError_t launch_slab(const Plan &plan, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream);
 int slab_max_coresident(const Plan &plan, int numCUs);
 int slab_columns();                          // x columns per slice
 int slab_max_slices();                       // largest P
 int slab_done_words();                       // words of a team's done array
+int slab_groups();                           // wave groups of a slice workgroup
+int slab_strips();                           // 64-column strips of a slice
 int slab_ring_slots();                       // exchange ring slots per team
 int slab_record_words();                     // tagged 8-byte words of a record
 int slab_bcast_words();                      // ... and of a broadcast block
@@ -264,6 +287,10 @@ hipError_t launch_stream_probe(const void *src, int64_t readBytes, void *dst, in
 // -1 if the plan has no strip kernel.
 int strip_max_coresident(const Plan &plan, int numCUs);
 
+// Wave groups of a slice workgroup of the strip kernel, and 64-column strips of
+// a slice.
+int strip_groups();
+int strip_strips();
 // Exchange ring slots per team of the strip kernel, and the tagged 8-byte
 // words of one exchange record (per slice) and of one broadcast block.
 int strip_ring_slots();

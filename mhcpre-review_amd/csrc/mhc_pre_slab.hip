@@ -16,7 +16,6 @@
 // strip w % 2 (64 columns of every stream) and belongs to group w / 2; group g
 // takes the team steps g, g + 4, ... (its own steps jj), so that four tiles
 // are in different phases on a CU and one group's exchange runs in the shadow
-// are in different phases on a CU and one group's exchange runs in the shadow
 // of the others' loads.  A wave keeps a ring of four tiles (16 rows x 6
 // streams x 64 columns, 48 VGPRs each).  Own step jj of a wave:
 //   1. the poll for the hPre of own tile jj - 2;
@@ -66,11 +65,13 @@
 // each has used the broadcasts up to m - 12 of its group, and m - 28 is the
 // same group's.
 //
-// Every wait on another workgroup is bounded.  A workgroup whose wait expires
+// Every wait on another workgroup is bounded.  A wave whose wait expires
 // (another kernel holds the CUs the rest of the grid needs) computes what it
-// was waiting for itself, from x, phi and gamma, and goes on alone: such a
-// launch is slow, never wrong and never stuck.  From then on it writes nothing
-// into the rings, whose slots are free only in the order above.
+// was waiting for itself, from x and the weights in the order of the exchange,
+// and goes on alone: such a launch is slow (6.3 ms at n = 6, D = 4096, T = 4096
+// with every wait expired) and its bits are the same.  From then on a slice's
+// wave writes nothing into the rings, whose slots are free only in the order
+// above.
 
 #include "mhc_pre_device.h"
 #include "mhc_pre_internal.h"
@@ -137,6 +138,8 @@ struct SlabArgs {
     uint64_t *bcast;  // [team][S] broadcast blocks
     uint64_t *done;   // [team][kMaxRest] words: the latest step a wave has finished reading
     LaunchTag tag;
+    char *hdr;        // workspace header: the status word
+    uint32_t launchId;
     int64_t T;
     int64_t D;
     int64_t K;
@@ -151,6 +154,7 @@ struct SlabArgs {
     float hcEps;
     float invFlatDim;
     uint32_t spinLimit;
+    uint32_t spinEvery;
 };
 
 // (Each phase of the kernel loads the arguments that it uses.)
@@ -182,17 +186,6 @@ __device__ __forceinline__ void store_exchange(const u32x4_t &v, __amdgpu_buffer
     }
 }
 
-// acc[i], i < 8
-__device__ __forceinline__ float pick8(const float (&acc)[9], int i)
-{
-    float v = acc[0];
-    static_for<7>([&](auto e) __attribute__((always_inline)) {
-        constexpr int k = decltype(e)::value + 1;
-        v = i == k ? acc[k] : v;
-    });
-    return v;
-}
-
 // ---------------------------------------------------------------------------
 // Reducer waves.  U: record loads in flight per lane (of a sum over the
 // slices).
@@ -221,7 +214,8 @@ struct Team {
     int64_t T;
     __device__ __forceinline__ Team(ArgsPtr ap, int t, int n, bool l, uint32_t e)
         : team(t), ntiles(n), P(ap->P), numTeams(ap->nGroups * ap->perGroup), local(l), epoch(e),
-          spinLimit(ap->spinLimit), recs(ap->recs + (size_t)t * kRingSlots * ap->P * Geo<N>::WORDS),
+          spinLimit(hurried(ap->spinEvery, blockIdx.x) ? 0u : ap->spinLimit),
+          recs(ap->recs + (size_t)t * kRingSlots * ap->P * Geo<N>::WORDS),
           flags(make_rsrc(ap->flags + (size_t)t * kRingSlots * ap->P * 2, kRingSlots * ap->P * 16)),
           done(make_rsrc(ap->done + (size_t)t * kMaxRest, kMaxRest * 8)), donePos((uint32_t)(t * kMaxRest)),
           invFlatDim(ap->invFlatDim), normEps(ap->normEps), T(ap->T)
@@ -301,6 +295,9 @@ __device__ __forceinline__ void crit_wave(ArgsPtr ap, const Team<N> &tm, int cls
                 }
             }
             if (expired || spins >= tm.spinLimit) {
+                if (!expired && lane == 0) {
+                    st_computed(ap->hdr, ap->launchId);
+                }
                 expired = true;
                 break;
             }
@@ -311,18 +308,15 @@ __device__ __forceinline__ void crit_wave(ArgsPtr ap, const Team<N> &tm, int cls
             sq.x = __shfl(acc.x, lane & 56);
             sq.y = __shfl(acc.y, lane & 56);
         } else {
-#pragma unroll 1
-            for (int r = 0; r < 16; ++r) {
-                float own[9];
-                own_sums<N, kBf16>(weights_of(ap), ap->x, ap->T, (int64_t)rt * 16 + r, 0, own);
-                if (rp == r >> 1) {
-                    const float v = pick8(own, ic - 1);
-                    acc.x = (r & 1) ? acc.x : v;
-                    acc.y = (r & 1) ? v : acc.y;
-                    sq.x = (r & 1) ? sq.x : own[8];
-                    sq.y = (r & 1) ? own[8] : sq.y;
-                }
-            }
+            f32x4_t v;  // lane (column, q): rows 4q .. + 3
+            float u;
+            group_sums<N, kBf16, false, kStrips>(weights_of(ap), tile_rsrc(ap->x, tm.T, (int)ap->K, rt), (int)ap->D,
+                                                 tm.P, lane & 15, 0, 1, v, u);
+            const int from = 16 * (rp >> 1) + (ic > 0 ? ic - 1 : 0);
+            const f32x4_t r4 = {__shfl(v[0], from), __shfl(v[1], from), __shfl(v[2], from), __shfl(v[3], from)};
+            acc = (rp & 1) ? make_float2(r4[2], r4[3]) : make_float2(r4[0], r4[1]);
+            sq.x = __shfl(u, 16 * (rp >> 1) + 2 * rp);
+            sq.y = __shfl(u, 16 * (rp >> 1) + 2 * rp + 1);
         }
         if (out) {
             u32x4_t wv;
@@ -402,6 +396,9 @@ __device__ __forceinline__ void rest_wave(ArgsPtr ap, const Team<N> &tm, int ru,
                 }
             }
             if (expired || spins >= tm.spinLimit) {
+                if (!expired && lane == 0) {
+                    st_computed(ap->hdr, ap->launchId);
+                }
                 expired = true;
                 break;
             }
@@ -418,21 +415,14 @@ __device__ __forceinline__ void rest_wave(ArgsPtr ap, const Team<N> &tm, int ru,
                 sq[e] = __shfl(acc[2 * (e & 1)], 56 + 2 * (quad & 3) + (e >> 1));
             }
         } else {
-#pragma unroll 1
-            for (int r = 0; r < 16; ++r) {
-#pragma unroll 1
-                for (int h = 0; h < 2; ++h) {  // columns first .. + 7, then + 6 .. + 13
-                    float own[9];
-                    own_sums<N, kBf16>(weights_of(ap), ap->x, ap->T, (int64_t)rt * 16 + r, first + 6 * h, own);
-                    const int i = lane % kRestCols - 6 * h;
-                    const float v = pick8(own, i & 7);
-                    const bool mine = quad == r >> 2 && i >= 0 && i < 8;
+            f32x4_t v;  // lane (column - first, q): rows 4q .. + 3
+            float u;
+            group_sums<N, kBf16, false, kStrips>(weights_of(ap), tile_rsrc(ap->x, tm.T, (int)ap->K, rt), (int)ap->D,
+                                                 tm.P, first + (lane & 15), 0, 1, v, u);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        acc[e] = mine && (r & 3) == e ? v : acc[e];
-                        sq[e] = quad == r >> 2 && (r & 3) == e ? own[8] : sq[e];
-                    }
-                }
+            for (int e = 0; e < 4; ++e) {
+                acc[e] = __shfl(v[e], 16 * (quad & 3) + lane % kRestCols);
+                sq[e] = __shfl(u, 20 * (quad & 3) + e);
             }
         }
         if (out) {
@@ -604,7 +594,7 @@ __global__ __launch_bounds__(kThreads) void slab_kernel(SlabArgs a)
     uint64_t *recsBase = la->recs + (size_t)team * kRingSlots * la->P * Z::WORDS;
     uint64_t *flagsBase = la->flags + (size_t)team * kRingSlots * la->P * 2;
     const int P32 = la->P;
-    const int spinLimit = (int)min(la->spinLimit, 0x7FFFFFFFu);
+    const int spinLimit = (int)min(hurried(la->spinEvery, g) ? 0u : la->spinLimit, 0x7FFFFFFFu);
     const __amdgpu_buffer_rsrc_t bcastAll =
         make_rsrc(la->bcast + (size_t)team * kRingSlots * Z::BWORDS, kRingSlots * Z::BWORDS * 8);
     const int nmine = (ntiles - grp4 + kGroups - 1) / kGroups;  // own steps (0 if none)
@@ -969,28 +959,13 @@ __global__ __launch_bounds__(kThreads) void slab_kernel(SlabArgs a)
     if (dead) {
         // A wait expired: this wave's hIn from that tile on, alone.
         const ArgsPtr ca = phase_args();
+        if (lane == 0) {
+            st_computed(ca->hdr, ca->launchId);
+        }
 #pragma unroll 1
-        for (int i = 16 * failFrom; i < 16 * nmine; ++i) {
-            const int64_t row = (int64_t)tile_of(i >> 4) * 16 + (i & 15);
-            if (row >= ca->T) {
-                break;
-            }
-            float own[9];
-            own_sums<N, kBf16>(weights_of(ca), ca->x, ca->T, row, 0, own);
-            const float ir = ref_inv_rms(own[8], ca->invFlatDim, ca->normEps);
-            const int c = col0 + lane;
-            float v = 0.f;
-#pragma unroll
-            for (int s = 0; s < N; ++s) {
-                const float pre = ref_sigmoid(own[s] * (ir * ca->alpha[0]), ca->bias[s], ca->hcEps);
-                if (c < Di) {
-                    const float prod = pre * x_to_f32<kBf16>(ca->x[row * Ki + s * Di + c]);
-                    v = s == 0 ? prod : v + prod;
-                }
-            }
-            if (c < Di) {
-                ca->hIn[row * Di + c] = (uint16_t)f32_to_x<kBf16>(v);
-            }
+        for (int i = failFrom; i < nmine; ++i) {
+            own_hin<N, kBf16, false, kStrips>(weights_of(ca), ca->x, ca->hIn, ca->alpha, ca->bias, ca->T, Di,
+                                              tile_of(i), ca->P, 1, col0, ca->invFlatDim, ca->normEps, ca->hcEps);
         }
     }
 }
@@ -1008,7 +983,7 @@ int slab_coresident_t(int numCUs)
 }
 
 template <int N, bool kBf16, bool kPrep>
-hipError_t launch_slab_t(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
+hipError_t launch_slab_t(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream)
 {
     char *ws = static_cast<char *>(workspace);
     SlabArgs a;
@@ -1027,6 +1002,8 @@ hipError_t launch_slab_t(const Plan &p, void *workspace, const LaunchTag &tag, h
     a.flags = reinterpret_cast<uint64_t *>(ws + p.wsSlabFlags);
     a.done = reinterpret_cast<uint64_t *>(ws + p.wsSlabDone);
     a.tag = tag;
+    a.hdr = ws;
+    a.launchId = launchId;
     a.T = p.T;
     a.D = p.D;
     a.K = p.K;
@@ -1041,6 +1018,7 @@ hipError_t launch_slab_t(const Plan &p, void *workspace, const LaunchTag &tag, h
     a.hcEps = p.hcEps;
     a.invFlatDim = p.invFlatDim;
     a.spinLimit = p.ownSpinLimit();
+    a.spinEvery = p.spinEvery;
     if (!p.fusedCooperative) {
         hipLaunchKernelGGL((slab_kernel<N, kBf16, kPrep>), dim3((unsigned)p.slab.grid), dim3(kThreads), 0,
                            stream, a);
@@ -1056,6 +1034,8 @@ hipError_t launch_slab_t(const Plan &p, void *workspace, const LaunchTag &tag, h
 int slab_columns() { return kCols; }
 int slab_max_slices() { return kMaxSlices; }
 int slab_done_words() { return kMaxRest; }
+int slab_groups() { return kGroups; }
+int slab_strips() { return kStrips; }
 int slab_ring_slots() { return kRingSlots; }
 int slab_record_words() { return Geo<6>::WORDS; }
 int slab_bcast_words() { return Geo<6>::BWORDS; }
@@ -1071,17 +1051,17 @@ int slab_max_coresident(const Plan &p, int numCUs)
     return p.isBf16 ? slab_coresident_t<6, true, false>(numCUs) : slab_coresident_t<6, false, false>(numCUs);
 }
 
-hipError_t launch_slab(const Plan &p, void *workspace, const LaunchTag &tag, hipStream_t stream)
+hipError_t launch_slab(const Plan &p, void *workspace, const LaunchTag &tag, uint32_t launchId, hipStream_t stream)
 {
     if (p.n != 6) {
         return hipErrorNotSupported;
     }
     if (p.bprep != nullptr) {
-        return p.isBf16 ? launch_slab_t<6, true, true>(p, workspace, tag, stream)
-                        : launch_slab_t<6, false, true>(p, workspace, tag, stream);
+        return p.isBf16 ? launch_slab_t<6, true, true>(p, workspace, tag, launchId, stream)
+                        : launch_slab_t<6, false, true>(p, workspace, tag, launchId, stream);
     }
-    return p.isBf16 ? launch_slab_t<6, true, false>(p, workspace, tag, stream)
-                    : launch_slab_t<6, false, false>(p, workspace, tag, stream);
+    return p.isBf16 ? launch_slab_t<6, true, false>(p, workspace, tag, launchId, stream)
+                    : launch_slab_t<6, false, false>(p, workspace, tag, launchId, stream);
 }
 
 }  // namespace mhc

@@ -122,6 +122,7 @@ struct StripArgs {
     float invFlatDim;
     uint32_t launchId;
     uint32_t spinLimit;
+    uint32_t spinEvery;
     LaunchTag tag;
 };
 
@@ -328,44 +329,38 @@ __device__ __forceinline__ void reducer_wg(int team, int ntiles, int r, int R,
     const float bias2 = first->bias[p2.c - 1];
     bool timedOut = false;
     // kOwn: the sums of mix columns j0 .. j1 - 1 (and, with j0 = 0, the sum of
-    // squares) of a tile whose records did not come, into group 0 of `sums`
-    // (the others zero), a wave per row.
+    // squares) of a tile whose records did not come, into `sums`: a wave takes
+    // one of the groups of slices and 16 columns at a time.
     const auto own_phase = [&](int rt, int j0, int j1) {
         const ArgsPtr a = late_args<StripArgs>();
         const int items = j0 == 0 ? Poll1::ITEMS : Poll2::ITEMS;
         const int groups = j0 == 0 ? Poll1::SG : Poll2::SG;
-        __syncthreads();
-        for (int i = tid; i < 2 * groups * items; i += kWaves * 64) {
-            sums[i] = 0.f;
-        }
+        const int rl = tid & 15;
+        const int grp = (tid & 63) >> 4;
         __syncthreads();
 #pragma unroll 1
-        for (int row = tid >> 6; row < 16; row += kWaves) {
-#pragma unroll 1
-            for (int j = j0; j < j1; j += 8) {
-                float own[9];
-                own_sums<N, kBf16>(WeightsRef{a->phi, a->gamma, a->bprep, (int)a->K}, a->x, a->T,
-                                   (int64_t)rt * 16 + row, j, own);
-                // Item (column j - j0) * 8 + row / 2 of the phase, component
-                // row % 2; the sum of squares is phase 1's last column.
-                const int at = 2 * (row >> 1) + (row & 1);
-                if ((tid & 63) == 0) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        if (j + i < j1) {
-                            sums[16 * (j + i - j0) + at] = own[i];
-                        }
-                    }
-                    if (j0 == 0) {
-                        sums[16 * N + at] = own[8];
-                    }
-                }
+        for (int u = tid >> 6; u < groups * ((j1 - j0 + 15) / 16); u += kWaves) {
+            const int j = j0 + 16 * (u / groups) + rl;
+            float *to = sums + 2 * items * (u % groups);
+            f32x4_t v;
+            float sq;
+            group_sums<N, kBf16, true, kStrips>(WeightsRef{a->phi, a->gamma, a->bprep, (int)a->K},
+                                                tile_rsrc(a->x, a->T, (int)a->K, rt), (int)a->D, P, j, u % groups,
+                                                groups, v, sq);
+            // Item (column j - j0) * 8 + row / 2 of the phase, component row % 2;
+            // the sum of squares is phase 1's last column.
+            if (j < j1) {
+                *reinterpret_cast<f32x4_t *>(&to[16 * (j - j0) + 4 * grp]) = v;
+            }
+            if (j0 == 0 && (rl >> 2) == grp) {
+                to[16 * N + rl] = sq;
             }
         }
         __syncthreads();
     };
     for (int k = r; k < ntiles; k += R) {
         const ArgsPtr a = late_args<StripArgs>();
+        const uint32_t limit = kOwn && hurried(a->spinEvery, blockIdx.x) ? 0u : a->spinLimit;
         const int rt = team + a->numTeams * k;
         const uint32_t slot = (uint32_t)(team * kRingSlots + k % kRingSlots);
         const __amdgpu_buffer_rsrc_t tr = make_rsrc(a->recs + (uint64_t)slot * P * RC::WORDS, P * RC::WORDS * 8);
@@ -386,9 +381,11 @@ __device__ __forceinline__ void reducer_wg(int team, int ntiles, int r, int R,
             if (timedOut) {
                 break;  // an earlier wait expired: no more waiting in this launch
             }
-            if (spins >= a->spinLimit) {
+            if (spins >= limit) {
                 if constexpr (!kOwn) {
                     record_timeout(a, tid);
+                } else if (tid == 0) {
+                    st_computed(a->hdr, a->launchId);
                 }
                 timedOut = true;
                 break;
@@ -474,9 +471,11 @@ __device__ __forceinline__ void reducer_wg(int team, int ntiles, int r, int R,
             if (timedOut) {
                 break;
             }
-            if (spins >= a->spinLimit) {
+            if (spins >= limit) {
                 if constexpr (!kOwn) {
                     record_timeout(a, tid);
+                } else if (tid == 0) {
+                    st_computed(a->hdr, a->launchId);
                 }
                 timedOut = true;
                 break;
@@ -532,7 +531,8 @@ __device__ __forceinline__ void reducer_wg(int team, int ntiles, int r, int R,
 
 // kOwn (D % 32 == 16): these widths ran kernels that wait for nobody before, so
 // a workgroup whose wait expires computes what it waited for itself, from x
-// and the weights, instead of writing NaN and reporting it.  One launch in
+// and the weights in the order of the exchange (the same bits), instead of
+// writing NaN and reporting it.  One launch in
 // place of three: D = 1200, T = 777 14.9 -> 12.5 us as an eager operator call,
 // D = 7056, T = 8192 266 -> 138 us.
 template <int N, bool kBf16, bool kPrep, bool kOwn>
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     uint64_t *bcastBase = a.bcast;
     uint64_t *statusW = reinterpret_cast<uint64_t *>(a.hdr);
     int P32 = a.P;
-    uint32_t spinLimit = a.spinLimit;
+    uint32_t spinLimit = kOwn && hurried(a.spinEvery, g) ? 0u : a.spinLimit;
     uint32_t launchId = a.launchId;
     asm volatile("" : "+s"(xBase), "+s"(hBase), "+s"(recsBase), "+s"(bcastBase), "+s"(statusW),
                  "+s"(P32), "+s"(spinLimit), "+s"(launchId));
@@ -1185,28 +1185,15 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     // outside the loop (kOwn: it computes its hIn from that tile on, alone).
     if constexpr (kOwn) {
         if (timedOut) {
+            if (lane == 0) {
+                st_computed(a.hdr, a.launchId);
+            }
+            constexpr int kGroups1 = ColPoll<N, 0, N + 1, 1>::SG;  // as the reducers add
 #pragma unroll 1
-            for (int i = 16 * failFrom; i < 16 * nmine; ++i) {
-                const int64_t row = (int64_t)tile_of(i >> 4) * 16 + (i & 15);
-                if (row >= T32) {
-                    break;
-                }
-                float own[9];
-                own_sums<N, kBf16>(WeightsRef{a.phi, a.gamma, a.bprep, Ki}, a.x, a.T, row, 0, own);
-                const float ir = ref_inv_rms(own[8], a.invFlatDim, a.normEps);
-                const int c = col0 + lane;
-                float v = 0.f;
-#pragma unroll
-                for (int s = 0; s < N; ++s) {
-                    const float pre = ref_sigmoid(own[s] * (ir * a.alpha[0]), a.bias[s], a.hcEps);
-                    if (c < Di) {
-                        const float prod = pre * x_to_f32<kBf16>(a.x[row * Ki + s * Di + c]);
-                        v = s == 0 ? prod : v + prod;
-                    }
-                }
-                if (c < Di) {
-                    a.hIn[row * Di + c] = (uint16_t)f32_to_x<kBf16>(v);
-                }
+            for (int i = failFrom; i < nmine; ++i) {
+                own_hin<N, kBf16, true, kStrips>(WeightsRef{a.phi, a.gamma, a.bprep, Ki}, a.x, a.hIn, a.alpha, a.bias,
+                                                 a.T, Di, tile_of(i), a.P, kGroups1, col0, a.invFlatDim, a.normEps,
+                                                 a.hcEps);
             }
         }
     } else if (timedOut && lane == 0) {
@@ -1244,6 +1231,7 @@ hipError_t launch_strip_t(const Plan &p, void *workspace, const LaunchTag &tag, 
     a.hPre = p.hasHPre ? p.hPre : nullptr;
     a.hdr = ws;
     a.tag = tag;
+    a.spinEvery = p.spinEvery;
     a.statusWord = p.statusWord;
     a.bcast = reinterpret_cast<uint64_t *>(ws + p.wsStripBcast);
     a.recs = reinterpret_cast<uint64_t *>(ws + p.wsStripRecs);
@@ -1303,6 +1291,8 @@ hipError_t launch_strip(const Plan &p, void *workspace, const LaunchTag &tag, ui
     });
 }
 
+int strip_groups() { return kGroups; }
+int strip_strips() { return kStrips; }
 int strip_ring_slots() { return kRingSlots; }
 
 int strip_record_words() { return Rec<4>::WORDS; }

@@ -61,28 +61,32 @@ def test_cell(pkg, orc, device, n, T, D, is_bf16, has_gamma, path, kernel):
     op.close()
 
 
+@pytest.mark.parametrize("knob", ["MHCPRE_SPIN_LIMIT=0", "MHCPRE_SPIN_EVERY=1", "MHCPRE_SPIN_EVERY=3"])
 @pytest.mark.parametrize("n,T,D,prepared", [(4, 40, 256, False), (6, 20, 528, True), (8, 19, 304, False)])
-def test_expired_waits_are_computed(pkg, orc, device, n, T, D, prepared):
+def test_expired_waits_are_computed(pkg, orc, device, n, T, D, prepared, knob):
     """A spin limit of 0 makes every wait that does not find its data at once
-    expire: the workgroups then compute the sums themselves, in the order of the
-    exchange (the same bits), and nothing is reported."""
+    expire, the other knob every wait of all or every third workgroup: they then
+    compute the sums themselves, in the order of the exchange (the same bits),
+    and it is no error."""
     x, phi, alpha, bias, gamma = _inputs(n, T, D, True, True)
     xt, pt, at, bt, gt = to_device(pkg, device, x, True, phi, alpha, bias, gamma)
     weights = pkg.MhcPreWeights(pt, gt, n) if prepared else None
     args = (xt, None, at, bt, None) if prepared else (xt, pt, at, bt, gt)
-    os.environ["MHCPRE_SPIN_LIMIT"] = "0"
+    name, value = knob.split("=")
+    os.environ[name] = value
     try:
         op = pkg.MhcPreOp(*args, h_pre=True, weights=weights)
     finally:
-        os.environ.pop("MHCPRE_SPIN_LIMIT", None)
-    want = run_gpu(pkg, device, x, True, phi, alpha, bias, gamma)
+        os.environ.pop(name, None)
+    want = run_gpu(pkg, device, x, True, phi, alpha, bias, gamma, kernel="cell")
     check(want, orc.mhc_pre(x, True, phi, alpha, bias, gamma), x, True, orc)
     for _ in range(2):
         for t in op.outputs():
             t.fill_(float("nan"))
-        _say(f"[cell] n={n} T={T} D={D} spin limit 0")
+        _say(f"[cell] n={n} T={T} D={D} {knob}")
         op.launch(check=True)
         assert op.kernel == "cell"
+        assert op.computed_waits() or name == "MHCPRE_SPIN_LIMIT"
         got = fetch(op)
         for k in got:
             assert np.array_equal(got[k], want[k]), k
@@ -110,5 +114,5 @@ def test_graph_replays_on_new_inputs(pkg, orc, device):
         torch.cuda.synchronize()
         check(fetch(op), orc.mhc_pre(xr, True, phi, alpha, bias, gamma), xr, True, orc)
         op.launch(check=True)
-        assert op.kernel == "cell"
+        assert op.kernel == "cell" and not op.computed_waits()
     op.close()

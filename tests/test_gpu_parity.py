@@ -54,7 +54,9 @@ def run_gpu(pkg, device, x_bits, is_bf16, phi, alpha, bias, gamma, norm_eps=1e-6
     op.launch()
     torch.cuda.synchronize()
     assert op.device_status() == 0
-    assert kernel is None or op.kernel == kernel
+    if kernel is not None:
+        assert op.kernel == kernel
+        assert not op.computed_waits()
     out = fetch(op)
     out["path"] = op.path
     op.close()

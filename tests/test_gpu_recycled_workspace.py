@@ -69,7 +69,7 @@ def test_header_restored_between_launches(pkg, orc, device, force, n, T, D, capt
         launch()
         torch.cuda.synchronize()
         _say(f"  launch {r}")
-        assert op.device_status() == 0 and op.kernel == force
+        assert op.device_status() == 0 and op.kernel == force and not op.computed_waits()
         check(fetch(op), orc.mhc_pre(x, True, *weights), x, True, orc)
     op.close()
 

@@ -84,32 +84,40 @@ def test_slab_prepared_matches_plain(pkg, orc, device, T, D, is_bf16):
     prep.close()
 
 
-@pytest.mark.parametrize("T,D,prepared", [(300, 528, False), (90, 1024, True)])
-def test_slab_expired_waits_are_computed(pkg, orc, device, T, D, prepared):
-    """A spin limit of 0 makes every wait that does not find its data at once
-    expire: the workgroups then compute what they waited for, the outputs are
-    right, nothing is reported, and the next launch on the workspace is too."""
-    x, phi, alpha, bias, gamma = _inputs(T, D, True, True)
-    xt, pt, at, bt, gt = to_device(pkg, device, x, True, phi, alpha, bias, gamma)
+@pytest.mark.parametrize("knob", ["MHCPRE_SPIN_LIMIT=0", "MHCPRE_SPIN_EVERY=5"])
+@pytest.mark.parametrize("T,D,is_bf16,prepared", [(300, 528, True, False), (90, 1024, True, True),
+                                                 (700, 1200, False, False), (170, 400, False, True)])
+def test_slab_expired_waits_are_computed(pkg, orc, device, T, D, is_bf16, prepared, knob):
+    """A spin limit of 0, in all or every fifth workgroup, makes every wait that
+    does not find its data at once expire: the workgroups then compute what they
+    waited for in the order of the exchange (the same bits), it is no error, and
+    the next launch on the workspace is clean."""
+    x, phi, alpha, bias, gamma = _inputs(T, D, is_bf16, True)
+    xt, pt, at, bt, gt = to_device(pkg, device, x, is_bf16, phi, alpha, bias, gamma)
     weights = pkg.MhcPreWeights(pt, gt, N) if prepared else None
     args = (xt, None, at, bt, None) if prepared else (xt, pt, at, bt, gt)
     os.environ["MHCPRE_FORCE_PATH"] = "slab"
-    os.environ["MHCPRE_SPIN_LIMIT"] = "0"
+    name, value = knob.split("=")
+    os.environ[name] = value
     try:
         hurried = pkg.MhcPreOp(*args, h_pre=True, weights=weights)
-        os.environ.pop("MHCPRE_SPIN_LIMIT")
+        os.environ.pop(name)
         calm = pkg.MhcPreOp(*args, h_pre=True, weights=weights, workspace=hurried.workspace)
     finally:
         os.environ.pop("MHCPRE_FORCE_PATH", None)
-        os.environ.pop("MHCPRE_SPIN_LIMIT", None)
-    ref = orc.mhc_pre(x, True, phi, alpha, bias, gamma)
+        os.environ.pop(name, None)
+    calm.launch(check=True)
+    want = fetch(calm)
+    check(want, orc.mhc_pre(x, is_bf16, phi, alpha, bias, gamma), x, is_bf16, orc)
     for op in (hurried, calm, hurried):
         for t in op.outputs():
             t.fill_(float("nan"))
-        _say(f"[slab] T={T} D={D} {'calm' if op is calm else 'spin limit 0'}")
+        _say(f"[slab] T={T} D={D} {'calm' if op is calm else knob}")
         op.launch(check=True)
-        assert op.kernel == "slab"
-        check(fetch(op), ref, x, True, orc)
+        assert op.kernel == "slab" and op.computed_waits() == (op is hurried)
+        got = fetch(op)
+        for k in got:
+            assert np.array_equal(got[k], want[k]), k
     hurried.close()
     calm.close()
 
@@ -133,7 +141,7 @@ def test_slab_graph_replays(pkg, orc, device):
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        assert op.kernel == "slab"
+        assert op.kernel == "slab" and not op.computed_waits()
         replayed = fetch(op)
         check(replayed, orc.mhc_pre(xs[i], True, phi, alpha, bias, gamma), xs[i], True, orc)
         op.launch(check=True)

@@ -59,28 +59,35 @@ def test_strip_at_half_step_widths(pkg, orc, device, T, D, is_bf16, has_gamma, p
     op.close()
 
 
-@pytest.mark.parametrize("T,D,prepared", [(300, 1200, False), (200, 720, True)])
-def test_expired_waits_are_computed(pkg, orc, device, T, D, prepared):
-    """A spin limit of 0 makes every wait that does not find its data at once
-    expire: the workgroups then compute what they waited for, the outputs are
-    right and nothing is reported."""
-    x, phi, alpha, bias, gamma = _inputs(T, D, True, True)
-    xt, pt, at, bt, gt = to_device(pkg, device, x, True, phi, alpha, bias, gamma)
+@pytest.mark.parametrize("knob", ["MHCPRE_SPIN_LIMIT=0", "MHCPRE_SPIN_EVERY=5"])
+@pytest.mark.parametrize("T,D,is_bf16,prepared", [(300, 1200, True, False), (200, 720, True, True),
+                                                 (500, 3600, False, False), (130, 240, False, True)])
+def test_expired_waits_are_computed(pkg, orc, device, T, D, is_bf16, prepared, knob):
+    """A spin limit of 0, in all or every fifth workgroup, makes every wait that
+    does not find its data at once expire: the workgroups then compute what they
+    waited for in the order of the exchange (the same bits) and it is no error."""
+    x, phi, alpha, bias, gamma = _inputs(T, D, is_bf16, True)
+    xt, pt, at, bt, gt = to_device(pkg, device, x, is_bf16, phi, alpha, bias, gamma)
     weights = pkg.MhcPreWeights(pt, gt, N) if prepared else None
     args = (xt, None, at, bt, None) if prepared else (xt, pt, at, bt, gt)
-    os.environ["MHCPRE_SPIN_LIMIT"] = "0"
+    name, value = knob.split("=")
+    os.environ[name] = value
     os.environ["MHCPRE_FORCE_PATH"] = "strip"
     try:
         op = pkg.MhcPreOp(*args, h_pre=True, weights=weights)
     finally:
-        os.environ.pop("MHCPRE_SPIN_LIMIT", None)
+        os.environ.pop(name, None)
         os.environ.pop("MHCPRE_FORCE_PATH", None)
-    ref = orc.mhc_pre(x, True, phi, alpha, bias, gamma)
+    want = run_gpu(pkg, device, x, is_bf16, phi, alpha, bias, gamma, force_path="strip", kernel="strip")
+    want.pop("path")
+    check(want, orc.mhc_pre(x, is_bf16, phi, alpha, bias, gamma), x, is_bf16, orc)
     for _ in range(2):
         for t in op.outputs():
             t.fill_(float("nan"))
-        _say(f"[strip half] T={T} D={D} spin limit 0")
+        _say(f"[strip half] T={T} D={D} {knob}")
         op.launch(check=True)
-        assert op.kernel == "strip"
-        check(fetch(op), ref, x, True, orc)
+        assert op.kernel == "strip" and op.computed_waits()
+        got = fetch(op)
+        for k in want:
+            assert np.array_equal(got[k], want[k]), k
     op.close()

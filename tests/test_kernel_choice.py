@@ -35,3 +35,12 @@ def _kernel(pkg, lib, **shape):
 ])
 def test_planned_kernel(pkg, lib, n, D, S, want):
     assert _kernel(pkg, lib, n=n, D=D, S=S) == want
+
+
+@pytest.mark.parametrize("n,D,S,want", [(6, 2000, 1 << 21, "slab"), (6, 2000, 1 << 23, "split"),
+                                        (4, 7056, 200000, "strip"), (4, 7056, 400000, "split"),
+                                        (4, 7168, 1 << 23, "strip")])
+def test_computing_an_expired_wait_is_bounded(pkg, lib, n, D, S, want):
+    """A slab or strip launch in place of kernels that wait for nobody has at
+    most 2^17 strips of rows per wave to compute alone (about a second)."""
+    assert _kernel(pkg, lib, n=n, D=D, S=S) == want
