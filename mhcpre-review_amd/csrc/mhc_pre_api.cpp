@@ -238,7 +238,11 @@ const char *test_env(const char *name);
 // 1x6x8 77.6, 1x7x3 77.7, 1x5x8 85.6, 1x7x2 86.7; D = 2048, T = 4096: 1x13x3
 // 43.9, 1x12x4 44.8, 1x14x2 44.9, 1x15x1 55.6, 8x1x4 56.1; D = 1024, T = 8192:
 // 1x25x2 43.8, 8x3x2 43.9, 1x23x3 46.6, 1x28x1 49.8, 8x3x1 52.3, 8x2x4 56.4; D
-// = 512, T = 8192: 1x42x2 30.8, 8x5x2 31.2, 8x4x4 33.8, 8x6x1 34.7.
+// = 512, T = 8192: 1x42x2 30.8, 8x5x2 31.2, 8x4x4 33.8, 8x6x1 34.7.  Where more
+// CUs are left over than the reducers of one team fewer need, three reducers
+// per team would not make up for it: T = 4096: D = 6144 1x4x4 116.1, 1x5x3 123.0
+// (1x4x8 118.6: four of them have no work and only hold their CUs), D = 7696
+// 1x3x4 174.5, 1x4x3 184.8, D = 8176 1x3x4 177.1, 1x3x8 180.4.
 mhc::SlabGeometry slab_geometry(int64_t D, int64_t T, const DeviceShape &s)
 {
     mhc::SlabGeometry best;
@@ -260,7 +264,8 @@ mhc::SlabGeometry slab_geometry(int64_t D, int64_t T, const DeviceShape &s)
         const double time = static_cast<double>((tiles + all - 1) / all) * step;
         if (best.P == 0 || time < bestTime * 0.999) {
             bestTime = time;
-            best = {P, groups, teams, R, CC, CR, s.cus, s.xcds};
+            // No more reducer workgroups than their waves have shares for (four).
+            best = {P, groups, teams, std::min(R, (CC + 3 * CR + 7) / 8), CC, CR, s.cus, s.xcds};
         }
     };
     const char *force = test_env("MHCPRE_SLAB");
