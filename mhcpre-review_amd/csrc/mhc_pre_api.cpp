@@ -323,6 +323,7 @@ int64_t cell_grid(int n, int64_t D, int64_t T, int strips)
 // D = 7168, T = 16 13.4 / 11.5.
 struct CellShape {
     int strips = 1;
+    int64_t grid = 0;
     bool faster = false;
 };
 CellShape cell_shape(int n, int64_t D, int64_t T)
@@ -336,11 +337,11 @@ CellShape cell_shape(int n, int64_t D, int64_t T)
         c.strips = std::atoi(forced) == 1 ? 1 : 2;
     }
     const int64_t columnTiles = (n * n + 2 * n + 15) / 16;
-    const int64_t grid = cell_grid(n, D, T, 2);
-    c.faster = c.strips == 1 || (grid > 0 && grid <= (P2 * columnTiles <= 64 ? 512 : 256));
+    const int64_t wide = cell_grid(n, D, T, 2);
+    c.grid = cell_grid(n, D, T, c.strips);
+    c.faster = c.grid > 0 && (c.strips == 1 || wide <= (P2 * columnTiles <= 64 ? 512 : 256));
     return c;
 }
-
 
 // Where the slab kernel is faster than the kernels of its shape's path (n = 6).
 // Measured on MI355X (bf16, gamma, back to back, us, slab / the rows or split
@@ -827,11 +828,10 @@ int validate_and_plan(const mhcTensor *x, const mhcTensor *phi, const mhcTensor 
     const bool cellForced = force != nullptr && std::strcmp(force, "cell") == 0;
     if (cellForced || force == nullptr) {
         const CellShape c = cell_shape(n, D, T);
-        const int64_t grid = cell_grid(n, D, T, c.strips);
-        if (cellForced ? grid > 0 : c.faster) {
+        if (cellForced ? c.grid > 0 : c.faster) {
             p.cellStrips = c.strips;
             p.cellP = static_cast<int>((D + 64 * c.strips - 1) / (64 * c.strips));
-            p.cellGrid = static_cast<int>(grid);
+            p.cellGrid = static_cast<int>(c.grid);
         }
     }
     // D % 32 == 16 (K % 128 != 0, the split path's shapes): the strip kernel in

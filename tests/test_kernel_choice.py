@@ -37,6 +37,15 @@ def test_planned_kernel(pkg, lib, n, D, S, want):
     assert _kernel(pkg, lib, n=n, D=D, S=S) == want
 
 
+@pytest.mark.parametrize("n,D,S,want", [(4, 7168, 8192, "strip"), (6, 4096, 4096, "slab"), (8, 16384, 64, "rows"),
+                                        (4, 256, 128, "cell")])
+def test_set_slice_width_keeps_to_the_grid(pkg, lib, monkeypatch, n, D, S, want):
+    """MHCPRE_CELL sets the cell kernel's slices where the kernel is made for
+    the grid that comes of it, and changes nothing elsewhere."""
+    monkeypatch.setenv("MHCPRE_CELL", "1")
+    assert _kernel(pkg, lib, n=n, D=D, S=S) == want
+
+
 @pytest.mark.parametrize("n,D,S,want", [(6, 2000, 1 << 21, "slab"), (6, 2000, 1 << 23, "split"),
                                         (4, 7056, 200000, "strip"), (4, 7056, 400000, "split"),
                                         (4, 7168, 1 << 23, "strip")])
