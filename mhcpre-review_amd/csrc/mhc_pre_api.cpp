@@ -1076,8 +1076,8 @@ int get_workspace(const mhcTensor *x, const mhcTensor *phi, const mhcTensor *alp
 
 // Co-resident workgroups of one of the executor's kernels on the
 // current device: the occupancy query runs once per process, device and
-// kernel instance (n, x dtype, prepared weights, slice width), and its
-// result is kept in the executor too.
+// kernel instance (n, x dtype, prepared weights, slice width, the strip kernel's
+// instance for D % 32 == 16), and its result is kept in the executor too.
 int cached_coresident(std::atomic<int> &slot, int (*query)(const mhc::Plan &, int),
                       const mhc::Plan &p, int cus)
 {
@@ -1090,11 +1090,11 @@ int cached_coresident(std::atomic<int> &slot, int (*query)(const mhc::Plan &, in
         (void)hipGetLastError();
         return query(p, cus);
     }
-    using Key = std::tuple<uintptr_t, int, int, bool, bool, int, int, int>;
+    using Key = std::tuple<uintptr_t, int, int, bool, bool, bool, int, int, int>;
     static std::mutex mu;
     static std::map<Key, int> known;
     const Key key{reinterpret_cast<uintptr_t>(query), device, p.n, p.isBf16, p.bprep != nullptr,
-                  p.fusedDw, p.cellStrips, cus};
+                  p.D % 32 != 0, p.fusedDw, p.cellStrips, cus};
     {
         std::lock_guard<std::mutex> lock(mu);
         const auto it = known.find(key);
