@@ -225,9 +225,8 @@ MHC_API int mhcPreGetWorkspaceSizePrepared(const mhcTensor *x, const mhcPreWeigh
  * MHC_STATUS_SCRATCH_TOO_SMALL (every workload up to n=4, D=7168, T=8192 and
  * n=8, D=8192, T=5472 fits).  All calls on one device share that device's
  * array: calls that overlap on a device (other streams, other host threads)
- * race and must be ordered by the caller.  An expired wait between
- * workgroups shows as NaN in the affected outputs (the status word lives in
- * the built-in array, which mhcPreQueryDeviceStatus does not read).
+ * race and must be ordered by the caller.  Expired waits are as mhcPre's
+ * (mhcPreQueryDeviceStatus reads the array's status word for a NULL workspace).
  */
 MHC_API int mhcPreNoAlloc(mhcPreExecutor *executor, hipStream_t stream);
 

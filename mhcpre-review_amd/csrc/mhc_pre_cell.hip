@@ -22,10 +22,10 @@
 // second read for hPost and hRes after hIn cost 2 us.
 //
 // Measured on MI355X (bf16, gamma, us per call back to back and in a graph of
-// calls; before: the two launches): n = 4, D = 256, T = 128 7.8 and 5.3, before
-// 10.6 and 7.5; n = 4, D = 7168, T = 16 8.0 and 7.5, before 10.4 and 8.6; n = 6,
-// D = 1024, T = 64 7.8 and 7.4, before 10.6 and 8.6; n = 8, D = 1024, T = 32 7.7
-// and 7.4, before 11.0 and 10.6.  What is left is the chain of launch, loads,
+// calls; before: the two launches): n = 4, D = 256, T = 128 7.1 and 5.5, before
+// 10.6 and 7.5; n = 4, D = 7168, T = 16 7.3 and 7.3, before 10.4 and 8.6; n = 6,
+// D = 1024, T = 64 7.1 and 7.0, before 10.6 and 8.6; n = 8, D = 1024, T = 32 7.2
+// and 7.2, before 11.0 and 10.6.  What is left is the chain of launch, loads,
 // record out and records in (an empty launch takes 2.5 to 3 us in a graph); the
 // bytes alone take under 1 us.
 //

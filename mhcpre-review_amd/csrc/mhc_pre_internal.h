@@ -7,7 +7,8 @@
 
 namespace mhc {
 
-// Kernel paths an executor can launch.
+// The path a shape belongs to: the kernels it runs, unless the cell, slab or
+// strip kernel runs in place of them (Plan::cellP, slab, stripInstead).
 enum class Path : int {
     kSplit = 0,   // prep B, split-K MFMA GEMM + sumsq partials, epilogue + hIn (x read twice)
     kFused = 1,   // one persistent kernel: x read once, kept in registers
@@ -18,7 +19,7 @@ enum class Path : int {
 // Device status word (first 8 bytes of the workspace): the low half holds a
 // code, the high half the host launch id of the launch that wrote it.  The
 // strip and fused kernels write (launch id, kDeviceTimeout) only when a wait
-// runs out, kernels that then compute what they waited for (launch id,
+// runs out, those that then compute what they waited for (launch id,
 // kDeviceComputed); the split path's first kernel writes kDeviceOk into the low
 // half.
 constexpr uint32_t kDeviceOk = 0u;

@@ -123,8 +123,8 @@ def test_slab_expired_waits_are_computed(pkg, orc, device, T, D, is_bf16, prepar
 
 
 def test_slab_graph_replays(pkg, orc, device):
-    """Replays of a captured launch with new x between them: the exchange epoch
-    is the workspace's, so no replay takes an earlier one's words."""
+    """Replays of a captured launch with new x between them: each counts itself
+    into the exchange's tags, so no replay takes an earlier one's words."""
     import torch
 
     T, D = 1200, 1024
