@@ -283,11 +283,9 @@ __device__ __forceinline__ const __attribute__((address_space(4))) Args *late_ar
     return p;
 }
 
-// The epoch of a launch, mixed into every exchange word's tag: the launch tag's
-// seed, and in a captured launch the replays this workgroup has counted in its
-// own word of the tag's.  One thread of every workgroup that the launch has
-// (spare ones too, the words stay equal) calls replay_load early and
-// launch_epoch once, later.
+// The epoch of a launch, mixed into every exchange word's tag (LaunchTag).  One
+// thread of every workgroup that the launch has (spare ones too, the words stay
+// equal) calls replay_load early and launch_epoch once, later.
 __device__ __forceinline__ uint32_t replay_load(uint32_t *words, int g)
 {
     return words == nullptr
@@ -303,8 +301,9 @@ __device__ __forceinline__ uint32_t launch_epoch(int g, uint32_t loaded)
     if (words == nullptr) {
         return a->tag.seed;
     }
-    __builtin_amdgcn_raw_buffer_store_b32(loaded + 1u, make_rsrc(words + g, 4), 0, 0, kCpolDev);
-    return a->tag.seed ^ mix32(loaded + 1u);
+    const uint32_t replay = (loaded + 1u) & 0x7FFFFFFFu;
+    __builtin_amdgcn_raw_buffer_store_b32(replay, make_rsrc(words + g, 4), 0, 0, kCpolDev);
+    return mix32(loaded >= kFilledNumbers ? loaded : a->tag.seed | (replay & ((1u << kReplayBits) - 1u)));
 }
 
 // Whether workgroup g is one that gives up its waits at once (Plan::spinEvery).

@@ -35,17 +35,25 @@ constexpr size_t kWsHeaderBytes = kWsReplayOff + 4 * kMaxExchangeGrid;
 
 // What the kernels whose workgroups exchange words (cell, slab, strip, fused)
 // mix into every tag, so that no word of another launch is taken for one of
-// this launch's, whatever the workspace held before: a hash of the launch's
-// number, which no two launches of a process share.  The replays of a captured
-// launch share it; `words` (null for an eager launch) then holds one word per
-// workgroup, equal in all of them, to which each replay adds one.
+// this launch's, whatever the workspace held before: the hash (mix32, a
+// bijection) of a number that no other launch of the process has.  An eager
+// launch: its own number, 31 bits of it (`seed`, hashed; `words` null).  The
+// replays of a captured launch share their arguments: it has a number among the
+// captured ones (`seed`, its upper 21 bits, 10 the highest two) and one word per
+// workgroup, equal in all of them, to which each replay adds one; the lower 11
+// bits are that count's, for a replay finds at its own places what the one
+// before it left there.  Without such words of its own, a node before the
+// launch sets words of the workspace to a whole number (11 the highest bits).
 struct LaunchTag {
     uint32_t seed = 0;
     uint32_t *words = nullptr;
 };
+constexpr uint32_t kCapturedNumbers = 0x80000000u;
+constexpr int kReplayBits = 11;
+constexpr uint32_t kFilledNumbers = 0xC0000000u;
 
-// The finalizer of MurmurHash3 (a bijection): distinct numbers, distinct
-// seeds, and the seeds of neighbouring launches differ in half their bits.
+// The finalizer of MurmurHash3: neighbouring numbers' hashes differ in half
+// their bits.
 __host__ __device__ inline uint32_t mix32(uint32_t v)
 {
     v ^= v >> 16;

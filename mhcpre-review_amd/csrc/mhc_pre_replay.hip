@@ -1,13 +1,12 @@
 // What tells the exchange words of one launch from those of every other: the
 // launch tag (see LaunchTag in mhc_pre_internal.h).
 //
-// An eager launch needs only its number, a kernel argument.  The replays of a
-// captured launch all carry the argument that was captured, so each captured
-// launch gets words of its own in a fixed array of the library's device code
-// object, one per workgroup, where every workgroup counts its replays.  They
-// are the only memory whose contents the exchange relies on: nobody else
-// writes them, all of a launch's words start equal and each replay adds one to
-// every one of them, so the workgroups of a replay agree whenever they start.
+// Each captured launch gets words of its own in a fixed array of the library's
+// device code object, one per workgroup, where every workgroup counts its
+// replays.  They are the only memory whose contents the exchange relies on:
+// nobody else writes them, all of a launch's words start equal and each replay
+// adds one to every one of them, so the workgroups of a replay agree whenever
+// they start.
 //
 // The words belong to the graph: a user object returns them when the graph and
 // everything made from it are gone.  A block is handed out again only for the
@@ -20,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
@@ -38,12 +38,13 @@ constexpr auto kRest = std::chrono::seconds(2);  // a returned block's replays m
 __device__ __align__(256) uint32_t replayWords[kReplayWords];
 __device__ uint32_t replayFills;
 
-// The n words of a launch without words of its own: a value that no fill had before.
+// The n words of a launch without words of its own: a number that no fill had before.
 __global__ __launch_bounds__(256) void fill_words(uint32_t *words, int n)
 {
     __shared__ uint32_t value;
     if (threadIdx.x == 0) {
-        value = __hip_atomic_fetch_add(&replayFills, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        value = kFilledNumbers |
+                __hip_atomic_fetch_add(&replayFills, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     for (int i = (int)threadIdx.x; i < n; i += 256) {
@@ -139,24 +140,30 @@ hipError_t replay_words_address(int device, uint32_t **ptr)
         return hipErrorInvalidValue;
     }
     Pools &all = pools();
-    std::lock_guard<std::mutex> lock(all.mu);
-    if (all.of[device].base == nullptr) {
-        // The caller has made `device` current: its copy of the array.
-        void *p = nullptr;
-        const hipError_t err = hipGetSymbolAddress(&p, HIP_SYMBOL(replayWords));
-        if (err != hipSuccess) {
-            return err;
-        }
-        all.of[device].base = static_cast<uint32_t *>(p);
+    {
+        std::lock_guard<std::mutex> lock(all.mu);
+        *ptr = all.of[device].base;
     }
-    *ptr = all.of[device].base;
+    if (*ptr != nullptr) {
+        return hipSuccess;
+    }
+    // The caller has made `device` current: its copy of the array.  (Not under
+    // the lock, which give_back takes inside calls of the runtime.)
+    void *p = nullptr;
+    const hipError_t err = hipGetSymbolAddress(&p, HIP_SYMBOL(replayWords));
+    if (err != hipSuccess) {
+        return err;
+    }
+    *ptr = static_cast<uint32_t *>(p);
+    std::lock_guard<std::mutex> lock(all.mu);
+    all.of[device].base = *ptr;
     return hipSuccess;
 }
 
 hipError_t make_launch_tag(uint32_t launchId, int device, int grid, void *workspace, hipStream_t stream,
                            LaunchTag &tag)
 {
-    tag.seed = mix32(launchId);
+    tag.seed = mix32(launchId & ~kCapturedNumbers);
     tag.words = nullptr;
     if (stream == nullptr) {
         return hipSuccess;  // (the null stream cannot be captured)
@@ -167,6 +174,8 @@ hipError_t make_launch_tag(uint32_t launchId, int device, int grid, void *worksp
     if (err != hipSuccess || status != hipStreamCaptureStatusActive) {
         return err;
     }
+    static std::atomic<uint32_t> captured{0};
+    tag.seed = kCapturedNumbers | ((captured.fetch_add(1u, std::memory_order_relaxed) << kReplayBits) & ~kFilledNumbers);
     uint32_t *base = nullptr;
     if (graph != nullptr && replay_words_address(device, &base) == hipSuccess) {
         if (Lease *lease = take(device, grid)) {

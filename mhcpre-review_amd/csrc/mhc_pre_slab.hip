@@ -9,7 +9,7 @@
 // (MFMA 1 us, the strips' meeting 0.7, hIn and the loads 1.4 per own step) and
 // the reducers bound it, not HBM (the same accesses without arithmetic: 5.7
 // TB/s).  Measured against the rows path's GEMM and second read of x: 96.9 ->
-// 71.1 us; D = 1024, T = 2048 26.0 -> 21.3 us (split path before).
+// 70.6 us; D = 1024, T = 2048 26.0 -> 21.4 us (split path before).
 //
 // Slice workgroup: 128 columns of each of the 6 streams (768 values of K),
 // whose B (144 KB) stays in LDS for the whole launch.  8 waves: wave w holds

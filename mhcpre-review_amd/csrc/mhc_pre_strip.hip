@@ -533,7 +533,7 @@ __device__ __forceinline__ void reducer_wg(int team, int ntiles, int r, int R,
 // a workgroup whose wait expires computes what it waited for itself, from x
 // and the weights in the order of the exchange (the same bits), instead of
 // writing NaN and reporting it.  One launch in
-// place of three: D = 1200, T = 777 16.0 -> 12.5 us as an eager operator call,
+// place of three: D = 1200, T = 777 16.0 -> 12.4 us as an eager operator call,
 // D = 7056, T = 8192 266 -> 138 us.
 template <int N, bool kBf16, bool kPrep, bool kOwn>
 __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
@@ -622,8 +622,16 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     const int p = role;
     const int strip = w & 3;
     const int half = w >> 2;  // the wave's group
-    const int Ki = (int)a.K;
-    const int Di = (int)a.D;
+    // The sizes the loop uses, as scalars of their own (as the other arguments
+    // below): left in the tuple they are loaded in, it is spilled and reloaded
+    // whole in each step of the fp16 instances (+3% at D = 7168, T = 8192).
+    // 32 bits hold them (the launch validates T < 2^31 / 16); byte offsets of a
+    // tile are formed in 64 bits.
+    int Ki = (int)a.K;
+    int Di = (int)a.D;
+    int T32 = (int)a.T;
+    int nTeams = (int)numTeams;
+    asm volatile("" : "+s"(Ki), "+s"(Di), "+s"(T32), "+s"(nTeams));
     const int col0 = p * kSlice + strip * kStripCols;
     // A strip past D (the last slice when D % 256 != 0) holds no columns:
     // its x reads zeros through size-0 resources, its B is zero and it
@@ -648,9 +656,6 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
         }
         return;
     }
-    // 32-bit tile and row indices (the launch validates T < 2^31 / 16);
-    // byte offsets of a tile are formed in 64 bits from them.
-    const int T32 = (int)a.T;
     // The kernel arguments the loop uses, as independent scalars: the
     // compiler otherwise keeps the argument block as one 16-register tuple
     // and spills and reloads it whole.
@@ -667,7 +672,6 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     const int nt32 = (int)ntiles;
     const int nmine = (nt32 - half + kGroups - 1) / kGroups;
     const int teamI = team;
-    const int nTeams = (int)numTeams;
     const uint32_t xTileBytes = 16u * (uint32_t)Ki * 2u;
     const uint32_t hTileBytes = 16u * (uint32_t)Di * 2u;
     // Team tile of own step jj, and its valid rows (0 past the last one).
@@ -1185,15 +1189,16 @@ __global__ __launch_bounds__(kWaves * 64) void strip_kernel(StripArgs a)
     // outside the loop (kOwn: it computes its hIn from that tile on, alone).
     if constexpr (kOwn) {
         if (timedOut) {
+            const ArgsPtr ca = late_args<StripArgs>();
             if (lane == 0) {
-                st_computed(a.hdr, a.launchId);
+                st_computed(ca->hdr, ca->launchId);
             }
             constexpr int kGroups1 = ColPoll<N, 0, N + 1, 1>::SG;  // as the reducers add
 #pragma unroll 1
             for (int i = failFrom; i < nmine; ++i) {
-                own_hin<N, kBf16, true, kStrips>(WeightsRef{a.phi, a.gamma, a.bprep, Ki}, a.x, a.hIn, a.alpha, a.bias,
-                                                 a.T, Di, tile_of(i), a.P, kGroups1, col0, a.invFlatDim, a.normEps,
-                                                 a.hcEps);
+                own_hin<N, kBf16, true, kStrips>(WeightsRef{ca->phi, ca->gamma, ca->bprep, Ki}, ca->x, ca->hIn,
+                                                 ca->alpha, ca->bias, ca->T, Di, tile_of(i), ca->P, kGroups1, col0,
+                                                 ca->invFlatDim, ca->normEps, ca->hcEps);
             }
         }
     } else if (timedOut && lane == 0) {
